@@ -49,6 +49,7 @@
 //    rounded to bf16 once, at the points the reference's bf16 autograd rounds;
 //    the outputs are bit-identical to torch._grouped_mm and its autograd on
 //    this GPU.
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 
@@ -907,70 +908,89 @@ static void launch_cfg(const GemmParams& p, int64_t R, hipStream_t stream) {
     hipLaunchKernelGGL((grouped_gemm_kernel<MODE, NW, WGM, TM, TN, NS, SKIP, OCC, ACT, false, BKT>), grid, block, 0, stream, p);
 }
 
-// Tile per mode (measured at the Kimi and DSv3 shapes). The forward modes run
-// 128 x 256 tiles, four waves, two workgroups per CU; gate_up over a long
-// contraction (D >= 4096) runs the same tile as eight 64 x 64 waves with 64-wide
-// k-steps (whole 128-byte rows per copy) and three stages at one workgroup per CU
-// (DSv3, D = 7168: 6.25 -> 5.46 ms; at D = 2304 it is 6 % slower). 256 x 256 tiles of
-// eight 64 x 128 waves with 64-wide k-steps, two stages, one workgroup per CU pay where
-// the experts are tall, from 512 rows per expert on average, with either epilogue: down
-// (Kimi, 512 rows: 0.81 -> 0.76-0.77 ms in the layer step; gpt-oss-20b, 2048 rows, H = 2880:
-// 1.21-1.23 -> 1.04-1.16 ms; at DSv3, 256 rows, 6 % slower) and gate_up (Kimi 1.58-1.59 ->
-// 1.54-1.55 ms in the layer step; 32K Kimi tokens, 1024 rows: 2.95 -> 2.72 ms; gpt-oss-20b
-// 2.55 -> 2.27-2.44 ms). Both 64-wide configurations run the software-pipelined
-// k-step (compute_ilv); down over a long contraction with short experts (H >= 2048,
-// DSv3) takes gate_up's long-contraction tile. dgu runs the
-// forward tile too: its epilogue reads g and u and writes dg and du, and with two
-// workgroups per CU one's epilogue overlaps the other's MFMAs (against one
-// eight-wave 128 x 512 workgroup: DSv3 3.15 -> 2.81 ms, Kimi -1.5 %). dx and dW run
-// one eight-wave workgroup per CU with three LDS stages and wider tiles, which
-// halves the copy traffic per flop of the dW operands: 128 x 384 (dx, D a multiple
-// of 384), 128 x 512 (dx, D a multiple of 512), 256 x 256 (dW). D and H are
-// multiples of 64 (check_gemm_shape). The tail skip is compiled into the
-// row-grouped modes except dx, whose second copy of the K loop costs more
-// registers than the skip saves.
+// Tile per mode. Workgroups are persistent and tiles cost about the same, so a launch
+// takes rounds = ceil(tiles / (CUs x workgroups per CU)) tile times, and which tile is
+// faster is decided by how its count divides the chip as much as by its own rate: at 640
+// tiles a tile with 512 slots runs two rounds, the second a quarter full. Each mode's
+// candidates carry the measured time of a round, in units of the 128 x 256 tile of eight
+// 64 x 64 waves at one workgroup per CU, and the smallest rounds x unit is launched.
+// Rounds use the expected m-tiles of a ragged routing: R / BM whole ones and half a tile
+// of remainder per expert, at least one for each expert that can have a row.
+// All candidates run the same MFMAs in the same k order: identical outputs.
+//
+//  gate_up, down   128 x 256, 64-wide k-steps, 3 stages        1.0
+//                  256 x 256, 64-wide k-steps, 2 stages        1.7 (gpt-oss gate_up 1.62)
+//  dgu             128 x 256, 32-wide, 3 stages                1.0
+//                  128 x 256 of four waves, 2 per CU           1.74 (512 slots)
+//                  64 x 256 of four waves, 3 stages, 2 per CU  1.45 (512 slots), where
+//                  an expert has more than one tile of rows (with fewer the weights'
+//                  bytes bound every tile)
+//  dx              128 x 256, 32-wide, 3 stages                1.0
+//                  128 x 384                                   1.45; 1.55 where no expert
+//                  has more than one tile of rows (the narrow tile streams weights faster)
+//                  128 x 512                                   1.73, where D is a multiple of
+//                  512 (its w1 half is parked in the dx rows: a partial tile wastes that
+//                  traffic too); the gpt-oss dx parks nothing and takes it at any D
+//                  128 x 256 of four waves, 2 per CU           1.95 (512 slots)
+//  dW              256 x 256, 32-wide, 3 stages; 128 x 128 of four waves, 2 per CU,
+//                  only where the wide tiles leave half the chip idle (the smaller tile
+//                  copies twice the bytes per flop: 382 -> 421 us at 1600 / 832 / 48 / 49152)
+//
+// Measured (us; D / H / experts / rows), against one fixed tile per mode with a bound on
+// the rows per expert: gate_up 2304 / 1024 / 256 / 512 399 -> 343, 16384 rows 580 -> 500,
+// 65536 950 -> 902; 7168 / 2048 / 32 / 16384 1043 -> 995; down 2048 / 1408 / 64 / 16384
+// 165 -> 128; dgu 2304 / 1024 / 256 / 16384 331 -> 289, 7168 / 2048 / 32 / 8199 458 ->
+// 400; dx 1024 / 704 / 64 / 16384 110 -> 90, 4096 / 1536 / 32 / 4096 233 -> 195; gpt-oss
+// 2880 / 2880 / 32 / 4096 gate_up 370 -> 284, down 230 -> 149, dgu 298 -> 206, dx 405 ->
+// 309; dW 256 / 512 / 8 / 8192 42 -> 24. The weights are read once whatever the tile: with
+// few rows per expert the eight-wave forward tile's three stages of whole 128-byte rows
+// keep more bytes in flight (5.2 -> 6.1 TB/s of weights at two rows per expert).
+static double rounds(double tiles, int per_cu) {
+  const double slots = (double)cu_count() * per_cu;
+  return tiles <= slots ? 1.0 : (double)((int64_t)((tiles + slots - 1.0) / slots));
+}
+static double expected_m_tiles(int64_t R, int64_t E, int bm) {
+  const double whole = (double)R / bm + 0.5 * (double)E, least = (double)(R < E ? R : E);
+  return whole > least ? whole : least;
+}
+
 template <int MODE, int ACT = kSwiGLU>
 static void launch_mode(const GemmParams& p, int64_t R, hipStream_t stream) {
+  auto n_tiles = [](int64_t n, int bn) { return (double)((n + bn - 1) / bn); };
+  const double m256 = expected_m_tiles(R, p.E, 256), m128 = expected_m_tiles(R, p.E, 128),
+               m64 = expected_m_tiles(R, p.E, 64);
   if constexpr (MODE == kFwdGateUp || MODE == kFwdDown) {
-    if constexpr (MODE == kFwdGateUp && ACT == kSwiGLU) {
-      if (p.D >= 4096) {  // long contractions: 128-byte rows per stage, eight 64 x 64 waves
-        launch_cfg<MODE, 8, 2, 4, 4, 3, true, 1, ACT, 64>(p, R, stream);
-        return;
-      }
-      if (R >= 512 * (int64_t)p.E) {  // tall experts: 256 x 256 tiles, whole 128-byte rows
-        launch_cfg<MODE, 8, 4, 4, 8, 2, true, 1, ACT, 64>(p, R, stream);
-        return;
-      }
-    }
-    if constexpr (MODE == kFwdGateUp && ACT == kOssGLU) {
-      if (R >= 512 * (int64_t)p.E) {  // tall experts (gpt-oss-20b: 2048 rows per expert)
-        launch_cfg<MODE, 8, 4, 4, 8, 2, true, 1, ACT, 64>(p, R, stream);
-        return;
-      }
-    }
-    if constexpr (MODE == kFwdDown && ACT == kSwiGLU) {
-      // short experts with a long contraction (DSv3: H = 2048, 256 rows per expert):
-      // gate_up's long-contraction tile (DSv3 down 2.72-2.74 -> 2.54-2.55 ms in the layer)
-      if (p.H >= 2048 && R < 512 * (int64_t)p.E) {
-        launch_cfg<MODE, 8, 2, 4, 4, 3, true, 1, ACT, 64>(p, R, stream);
-        return;
-      }
-    }
-    if constexpr (MODE == kFwdDown) {
-      if (R >= 512 * (int64_t)p.E) {  // tall experts
-        launch_cfg<MODE, 8, 4, 4, 8, 2, true, 1, ACT, 64>(p, R, stream);
-        return;
-      }
-    }
-    launch_cfg<MODE, 4, 2, 4, 8, 2, true, 2, ACT>(p, R, stream);
+    const double nt = n_tiles(MODE == kFwdGateUp ? 2 * (int64_t)p.H : p.D, 256);
+    const double tall = MODE == kFwdGateUp && ACT == kOssGLU ? 1.62 : 1.7;
+    if (tall * rounds(m256 * nt, 1) < rounds(m128 * nt, 1))
+      launch_cfg<MODE, 8, 4, 4, 8, 2, true, 1, ACT, 64>(p, R, stream);
+    else
+      launch_cfg<MODE, 8, 2, 4, 4, 3, true, 1, ACT, 64>(p, R, stream);
   } else if constexpr (MODE == kBwdDgu) {
-    launch_cfg<MODE, 4, 2, 4, 8, 2, true, 2, ACT>(p, R, stream);
+    const double nt = n_tiles(p.H, 256);
+    const double c_one = rounds(m128 * nt, 1), c_two = 1.74 * rounds(m128 * nt, 2),
+                 c_low = 1.45 * rounds(m64 * nt, 2);
+    const bool several = m64 > (double)(R < p.E ? R : p.E);
+    if (several && c_low < c_one && c_low < c_two) launch_cfg<MODE, 4, 1, 4, 4, 3, true, 2, ACT>(p, R, stream);
+    else if (c_two < c_one) launch_cfg<MODE, 4, 2, 4, 8, 2, true, 2, ACT>(p, R, stream);
+    else launch_cfg<MODE, 8, 2, 4, 4, 3, true, 1, ACT>(p, R, stream);
   } else if constexpr (MODE == kBwdDx) {
-    if (p.D % 384 == 0) launch_cfg<MODE, 8, 2, 4, 6, 3, false, 1, ACT>(p, R, stream);
-    else if (p.D % 512 == 0) launch_cfg<MODE, 8, 2, 4, 8, 3, false, 1, ACT>(p, R, stream);
+    const bool several = m128 > (double)(R < p.E ? R : p.E);
+    const double c256 = rounds(m128 * n_tiles(p.D, 256), 1),
+                 c384 = (several ? 1.45 : 1.55) * rounds(m128 * n_tiles(p.D, 384), 1),
+                 c512 = ACT == kOssGLU || p.D % 512 == 0 ? 1.73 * rounds(m128 * n_tiles(p.D, 512), 1) : INFINITY,
+                 c_two = 1.95 * rounds(m128 * n_tiles(p.D, 256), 2);
+    const double best = fmin(fmin(c256, c384), fmin(c512, c_two));
+    if (best == c384) launch_cfg<MODE, 8, 2, 4, 6, 3, false, 1, ACT>(p, R, stream);
+    else if (best == c512) launch_cfg<MODE, 8, 2, 4, 8, 3, false, 1, ACT>(p, R, stream);
+    else if (best == c256) launch_cfg<MODE, 8, 2, 4, 4, 3, false, 1, ACT>(p, R, stream);
     else launch_cfg<MODE, 4, 2, 4, 8, 2, false, 2, ACT>(p, R, stream);
   } else {
-    launch_cfg<MODE, 8, 4, 4, 8, 3, false, 1, kSwiGLU>(p, R, stream);
+    const int64_t m = MODE == kBwdDw13 ? 2 * (int64_t)p.H : p.D, n = MODE == kBwdDw13 ? p.D : p.H;
+    if (2 * p.E * n_tiles(m, 256) * n_tiles(n, 256) <= cu_count())
+      launch_cfg<MODE, 4, 2, 4, 4, 3, false, 2, kSwiGLU>(p, R, stream);
+    else
+      launch_cfg<MODE, 8, 4, 4, 8, 3, false, 1, kSwiGLU>(p, R, stream);
   }
 }
 
