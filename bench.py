@@ -108,7 +108,8 @@ PEAK_FP32_TFLOPS = 157.3  # MI355X dense fp32 MFMA
 
 GEMM_ENTRIES = tuple(f"moe_{kind}_{m}" for kind in ("grouped_gemm", "fp8_gemm", "mxfp8_gemm", "grouped_gemm_oss",
                                                    "grouped_gemm_f32")
-                     for m in ("gate_up", "down", "bwd_dgu", "bwd_dx", "bwd_dw13", "bwd_dw1", "bwd_dw2", "bwd_dw"))
+                     for m in ("gate_up", "down", "bwd_dgu", "bwd_dx", "bwd_dw13", "bwd_dw1", "bwd_dw2", "bwd_dw",
+                               "bwd_dw_all"))
 
 
 def kernel_work(name: str, w: dict) -> tuple[str, float]:
@@ -120,9 +121,9 @@ def kernel_work(name: str, w: dict) -> tuple[str, float]:
     r = n * k
     b = 4 if w.get("fp32") else 2  # row bytes per element (fp32 activations on the c1 workloads)
     sb = w.get("score_before", True)
-    # bwd_dw (fp32 kernels) is one launch per weight: 2 R D H each
+    # bwd_dw (fp32 kernels) is one launch per weight: 2 R D H each; bwd_dw_all all three
     flops = {"gate_up": 4, "down": 2, "bwd_dgu": 2, "bwd_dx": 4, "bwd_dw13": 4, "bwd_dw1": 4, "bwd_dw2": 2,
-             "bwd_dw": 2}
+             "bwd_dw": 2, "bwd_dw_all": 6}
     for kind in ("moe_grouped_gemm_oss_", "moe_grouped_gemm_f32_", "moe_grouped_gemm_", "moe_fp8_gemm_",
                  "moe_mxfp8_gemm_"):
         if name.startswith(kind) and name[len(kind):] in flops:

@@ -266,6 +266,19 @@ int moe_grouped_gemm_f32_bwd_dx(const float* dg, const float* du, const float* w
 int moe_grouped_gemm_f32_bwd_dw(const float* a, const float* b, const int64_t* counts, int64_t n_rows,
                                 int32_t n_experts, int32_t m, int32_t n, float* out, moe_stream_t stream);
 
+/* Zeroes the rows from sum(counts) on (counts clamped to [0, n_rows]) of up to four
+ * fp32 tensors [n_rows, cols]; cols 0: none. */
+int moe_zero_rows_past_f32(const int64_t* counts, int64_t n_rows, int32_t n_experts, float* t0, int64_t cols0,
+                           float* t1, int64_t cols1, float* t2, int64_t cols2, float* t3, int64_t cols3,
+                           moe_stream_t stream);
+
+/* All three weight gradients in one launch: dw1 = dg^T x, dw3 = du^T x [E, H, D],
+ * dw2 = dy^T h [E, D, H], each as moe_grouped_gemm_f32_bwd_dw gives it. */
+int moe_grouped_gemm_f32_bwd_dw_all(const float* dg, const float* du, const float* dy, const float* x,
+                                    const float* h, const int64_t* counts, int64_t n_rows, int32_t n_experts,
+                                    int32_t dim, int32_t hidden, float* dw1, float* dw3, float* dw2,
+                                    moe_stream_t stream);
+
 /* ---------------------------------------------------------------------------
  * gpt-oss experts (torchtitan/models/gpt_oss/moe.py:43-52, 92-122, the
  * grouped-mm path): mlp1_weight [E, 2H, D] bf16 with the glu row 2j and the

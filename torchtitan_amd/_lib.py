@@ -53,6 +53,8 @@ SIGNATURES: dict[str, list] = {
     "moe_grouped_gemm_f32_bwd_dgu": [P, P, P, P, P, I64, I32, I32, I32, P, P, P],
     "moe_grouped_gemm_f32_bwd_dx": [P, P, P, P, P, I64, I32, I32, I32, P, P],
     "moe_grouped_gemm_f32_bwd_dw": [P, P, P, I64, I32, I32, I32, P, P],
+    "moe_zero_rows_past_f32": [P, I64, I32, P, I64, P, I64, P, I64, P, I64, P],
+    "moe_grouped_gemm_f32_bwd_dw_all": [P, P, P, P, P, P, I64, I32, I32, I32, P, P, P, P],
     "moe_fp8_padded_rows": [I64, I32],
     "moe_fp8_quant_rows": [P, I64, I32, P, P, P],
     "moe_fp8_quant_cols_t": [P, I32, I32, I32, P, I64, I64, P, I64, P],

@@ -12,34 +12,52 @@
 //   bwd_dx   dx = dg w1 + du w3
 //   bwd_dw   out[e] = a_e^T b_e over expert e's rows (dw1, dw3, dw2)
 //
-// Tiles: 64 x 64 outputs per 256-thread workgroup, 16 of k per LDS stage, each
-// wave a 32 x 32 quarter as 2 x 2 MFMA tiles. Operands are staged k-major in
-// LDS (rows padded to 80 floats, so the 16-lane column reads of one k-row and
-// the 64-lane scalar stores of one k-row are both free of bank conflicts).
-// The next stage is loaded into registers while the current one computes.
-// Row-grouped modes map blockIdx.x to (expert, 64-row tile) from a scan of the
-// counts in LDS, so no host sync or padding is needed; surplus blocks exit.
+// Tiles: 64 x 64 outputs, 32 of k per LDS stage, two stages; eight waves per workgroup in
+// the row modes, four in dW. What bounds fp32 is the matrix cores (a 16 x 16 x 4 MFMA
+// takes 32 clocks; 154 TFLOP/s measured over a large product) and, at few tiles, how
+// evenly 64 x 64 tiles fall on the CUs, so the rest has to stay out of their way:
+// operands go to LDS by direct-to-LDS copies (16 bytes a lane, no staging registers or
+// LDS stores), and every LDS read is one 8- or 16-byte read that feeds two or four MFMAs.
+// Which k a lane group supplies to an MFMA is free as long as both operands agree: step
+// (h, j) takes k = 16 h + 4 g + j from lane group g = lane / 16, so that
+//  * a k-contiguous operand (rows of 128 bytes, 16-byte chunk c of row r at c ^ (r & 7))
+//    gives a lane the operands of four steps in one 16-byte read of its row;
+//  * a k-major operand (32 k-rows of 64 columns, chunk c of k-row k at
+//    c ^ 8 ((k >> 2) & 1)) gives a lane two neighbouring columns of its k, which go to two
+//    MFMA tiles: tile q holds columns 2 i + q, and a lane's results over the tiles are
+//    contiguous in the output row.
+// All of these reads are free of bank conflicts.
+// Measured (us, against scalar LDS reads of register-staged 16-deep tiles, four waves) at
+// 8192 rows of 8 experts, dim 256, hidden 512 | 16384 rows, 512, 1024: gate_up 59 -> 57 |
+// 330 -> 313, down 36 -> 32 | 186 -> 164, dgu 39 -> 34 | 224 -> 184, dx 64 -> 62 | 350 ->
+// 343, the three dW (one launch, before three) 123 -> 72 | 592 -> 498. Without copies and
+// stores gate_up still takes 43 | 264 us: the MFMAs at the clock they leave. Three stages
+// measured the same as two.
+// Row-grouped modes map workgroups to (expert, 64-row tile) from a scan of the counts,
+// so no host sync or padding is needed; surplus workgroups exit.
 #include "common.h"
 
 namespace moe {
 namespace f32g {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+#define LDSP __attribute__((address_space(3)))
 
 constexpr int kMaxE = 1024;
-constexpr int BM = 64, BN = 64, BK = 16;
-constexpr int LDS_ROW = 80;  // floats per k-row of a staged tile
+constexpr int BM = 64, BN = 64, BK = 32;
+constexpr int kTile = 64 * BK;  // floats of one operand's stage (8 KB)
 
-enum Mode : int { kGateUp = 0, kDown = 1, kDgu = 2, kDx = 3, kDw = 4 };
+enum Mode : int { kGateUp = 0, kDown = 1, kDgu = 2, kDx = 3 };
 
 struct Params {
   const int64_t* counts;
   int64_t R;
   int E;
-  int N, K;        // row modes: N output columns, K contraction; dW: M = K (a's columns), N (b's columns)
-  const float* a;  // row operand [R, K] (dW: [R, M])
+  int N, K;        // N output columns, K contraction (dx: of each half)
+  const float* a;  // row operand [R, K]
   const float* a2; // second row operand (dx: du)
-  const float* b;  // NT: [E, N, K]; NN: [E, K, N]; dW: [R, N]
+  const float* b;  // NT: [E, N, K]; NN: [E, K, N]
   const float* b2; // second weight (gate_up: w3; dx: w3)
   const float* g;  // dgu: saved g, u [R, N]
   const float* u;
@@ -50,55 +68,333 @@ struct Params {
 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
 
-// expert e's segment: rows [start, start + count) clamped to R; tiles of 64 rows
-struct Seg {
-  int64_t start;
-  int count;
-  int tile;  // first 64-row tile of the expert (row modes)
-};
+__device__ const float4 kZeroChunk[4] = {};  // source of the k-rows past a segment
 
-// Which expert (and 64-row tile within it) block `bx` computes; e = -1 when bx
-// is past the last tile. Every thread of the block must call it.
-__device__ __forceinline__ void find_tile(const Params& p, int bx, int* s_tmp, int* s_out, int& e, Seg& seg,
-                                          int& mt) {
-  int cnt[4], tiles[4], st[4], tst[4];
+// global accesses of four floats: any tensor of floats, 16-byte aligned or not
+typedef f32x4_t f32x4_u __attribute__((aligned(4)));
+
+// lane i's 16 bytes at g land at LDS byte address lds + 16 i: a direct-to-LDS copy, or,
+// where an operand is not 16-byte aligned, through registers
+template <bool ALIGNED>
+__device__ __forceinline__ void copy16(const float* g, uint32_t lds) {
+  if constexpr (ALIGNED)
+    asm volatile("global_load_lds_dwordx4 %0, off" :: "v"(g), "{m0}"(lds) : "memory");
+  else
+    *(LDSP f32x4_t*)(size_t)(lds + 16 * (threadIdx.x & 63)) = *(const f32x4_u*)g;
+}
+__device__ __forceinline__ uint32_t lds_addr(float* p) { return (uint32_t)(size_t)((LDSP float*)p); }
+
+// Expert segments: rows [start, start + count) clamped to R.
+struct Seg { int start, count; };
+
+// This lane's experts 4 t .. 4 t + 3 of the counts (t = threadIdx.x) with their starts,
+// counts cut where they run past R.
+__device__ __forceinline__ void scan_counts(const int64_t* counts, int64_t R, int E, int* s_tmp, int (&st)[4],
+                                            int (&cnt)[4]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int ee = threadIdx.x * 4 + i;
-    const int64_t c = ee < p.E ? p.counts[ee] : 0;
-    cnt[i] = c < 0 ? 0 : (int)(c > p.R ? p.R : c);
+    const int64_t c = ee < E ? counts[ee] : 0;
+    cnt[i] = c < 0 ? 0 : (int)(c > R ? R : c);
   }
   block_exclusive_scan4(cnt, st, s_tmp);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    // clamp the segment to R (counts that sum past R are cut at R)
-    const int64_t room = p.R - st[i];
+    const int64_t room = R - st[i];
     cnt[i] = room <= 0 ? 0 : (cnt[i] > room ? (int)room : cnt[i]);
-    tiles[i] = (cnt[i] + BM - 1) / BM;
   }
-  block_exclusive_scan4(tiles, tst, s_tmp);
-  if (threadIdx.x == 0) s_out[0] = -1;
-  __syncthreads();
+}
+
+// The expert and 64-row tile of workgroup tile `bx`; e = -1 past the last tile. Every
+// thread of the block must call it.
+__device__ __forceinline__ void find_tile(const Params& p, int bx, int* s_tmp, int* s_out, int& e, Seg& seg, int& mt) {
+  int cnt[4], st[4], tiles[4], tst[4];
+  scan_counts(p.counts, p.R, p.E, s_tmp, st, cnt);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) tiles[i] = (cnt[i] + BM - 1) / BM;
+  const int total = block_exclusive_scan4(tiles, tst, s_tmp);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int ee = threadIdx.x * 4 + i;
-    if (ee < p.E && tiles[i] > 0 && bx >= tst[i] && bx < tst[i] + tiles[i]) {
+    if (ee < p.E && bx >= tst[i] && bx < tst[i] + tiles[i]) {
       s_out[0] = ee;
       s_out[1] = st[i];
       s_out[2] = cnt[i];
       s_out[3] = tst[i];
     }
   }
+  if (bx >= total && threadIdx.x == 0) s_out[0] = -1;
   __syncthreads();
   e = s_out[0];
   seg.start = s_out[1];
   seg.count = s_out[2];
-  seg.tile = s_out[3];
-  mt = bx - seg.tile;
+  mt = bx - s_out[3];
 }
 
 // dW: start and count of expert e's rows
-__device__ __forceinline__ void find_segment(const Params& p, int e, int* s_tmp, int* s_out, Seg& seg) {
+__device__ __forceinline__ void find_segment(const int64_t* counts, int64_t R, int E, int e, int* s_tmp, int* s_out,
+                                             Seg& seg) {
+  int cnt[4], st[4];
+  scan_counts(counts, R, E, s_tmp, st, cnt);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if ((int)threadIdx.x * 4 + i == e) {
+      s_out[0] = st[i];
+      s_out[1] = cnt[i];
+    }
+  }
+  __syncthreads();
+  seg.start = s_out[0];
+  seg.count = s_out[1];
+}
+
+// A wave copies two of an operand's eight 1 KB pieces (8 rows, or 4 k-rows) of a stage.
+// k-contiguous: lane -> row 8 c + lane / 8, 16-byte chunk (lane & 7) ^ (row & 7)
+__device__ __forceinline__ int row_of(int c, int lane) { return 8 * c + (lane >> 3); }
+__device__ __forceinline__ int row_chunk(int lane) { return (lane & 7) ^ ((lane >> 3) & 7); }
+// k-major: lane -> k-row 4 c + lane / 16, chunk (lane & 15) ^ 8 ((k >> 2) & 1), k >> 2 == c
+__device__ __forceinline__ int krow_of(int c, int lane) { return 4 * c + (lane >> 4); }
+__device__ __forceinline__ int krow_chunk(int c, int lane) { return (lane & 15) ^ ((c & 1) << 3); }
+
+// chunk h of a k-contiguous tile's row: steps (h, 0 .. 3) of lane group g
+__device__ __forceinline__ f32x4_t read_row(const float* tile, int row, int g, int h) {
+  return *(const f32x4_t*)(tile + row * BK + (((g + 4 * h) ^ (row & 7)) << 2));
+}
+// step (h, j) of a k-major tile: columns 32 w + 2 (lane & 15), + 1
+__device__ __forceinline__ f32x2_t read_col2(const float* tile, int lane, int w, int h, int j) {
+  const int g = lane >> 4, k = 16 * h + 4 * g + j;
+  const int c = 8 * w + ((lane & 15) >> 1);
+  return *(const f32x2_t*)(tile + k * 64 + ((c ^ ((g & 1) << 3)) << 2) + 2 * (lane & 1));
+}
+
+// Consecutive workgroups of one XCD take neighbouring tiles (they share an operand in its L2).
+__device__ __forceinline__ int xcd_order() {
+  const int G = gridDim.x, b = blockIdx.x;
+  return G % 8 == 0 ? (b & 7) * (G >> 3) + (b >> 3) : b;
+}
+
+// Row-grouped modes: 64 rows of one expert x 64 output columns. Waves: 32 x 32 each where
+// the weights are k-contiguous (gate_up, down), 16 x 64 where they are k-major (dgu, dx).
+template <int MODE, bool ALIGNED>
+__global__ __launch_bounds__(512, MODE == kGateUp ? 6 : 8) void rows_kernel(Params p) {
+  constexpr bool kTwoB = MODE == kGateUp;                 // two weights into two accumulator sets
+  constexpr bool kNT = MODE == kGateUp || MODE == kDown;  // weights [E, N, K]; else [E, K, N]
+  constexpr int TN = 2, NB = kTwoB ? 2 : 1;
+  __shared__ __attribute__((aligned(1024))) float sA[2][kTile];
+  __shared__ __attribute__((aligned(1024))) float sB[2][NB][kTile];
+  __shared__ int s_tmp[8];
+  __shared__ int s_out[4];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ntn = p.N / BN, t = xcd_order();
+  int e, mt;
+  Seg seg;
+  find_tile(p, t / ntn, s_tmp, s_out, e, seg, mt);
+  const int n0 = (t % ntn) * BN;
+  if (e < 0) return;  // past the last tile
+  const int64_t row0 = (int64_t)seg.start + (int64_t)mt * BM;
+  const int nrows = min(BM, seg.count - mt * BM);
+  const int wm = w >> 1, wn = w & 1;
+  const int g = lane >> 4, li = lane & 15;
+
+  // this lane's copy sources: rows past the segment re-read its last row (their results
+  // are not stored)
+  const float *srcA, *srcB[NB];
+  srcA = p.a + (row0 + min(row_of(w, lane), nrows - 1)) * p.K + row_chunk(lane) * 4;
+#pragma unroll
+  for (int q = 0; q < NB; ++q) {
+    const float* base = (q ? p.b2 : p.b) + (int64_t)e * p.N * p.K;
+    srcB[q] = kNT ? base + (int64_t)(n0 + row_of(w, lane)) * p.K + row_chunk(lane) * 4
+                  : base + (int64_t)krow_of(w, lane) * p.N + n0 + krow_chunk(w, lane) * 4;
+  }
+  const int64_t stepB = kNT ? BK : (int64_t)BK * p.N;
+  const int nk = p.K / BK, nkt = MODE == kDx ? 2 * nk : nk;
+  // dx: the second half of the k-steps runs over du and w3
+  const int64_t jumpA = MODE == kDx ? p.a2 - p.a : 0, jumpB = MODE == kDx ? p.b2 - p.b : 0;
+  auto issue = [&](int kt, int s) {
+    const bool half = MODE == kDx && kt >= nk;
+    const int kk = half ? kt - nk : kt;
+    copy16<ALIGNED>(srcA + (half ? jumpA : 0) + kk * BK, lds_addr(sA[s] + w * 256));
+#pragma unroll
+    for (int q = 0; q < NB; ++q)
+      copy16<ALIGNED>(srcB[q] + (half ? jumpB : 0) + kk * stepB, lds_addr(sB[s][q] + w * 256));
+  };
+
+  f32x4_t acc[NB][TN];
+#pragma unroll
+  for (int q = 0; q < NB; ++q)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[q][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  issue(0, 0);
+  for (int kt = 0; kt < nkt; ++kt) {
+    const int s = kt & 1;
+    // the stage has landed in every wave, and every wave is done with the other buffer
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kt + 1 < nkt) issue(kt + 1, s ^ 1);
+    const float* cA = sA[s];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32x4_t av = read_row(cA, 16 * wm + li, g, h);
+      if constexpr (kNT) {
+        f32x4_t bv[NB][TN];
+#pragma unroll
+        for (int q = 0; q < NB; ++q)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) bv[q][j] = read_row(sB[s][q], 32 * wn + 16 * j + li, g, h);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int q = 0; q < NB; ++q)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              acc[q][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[q][j][v], av[v], acc[q][j], 0, 0, 0);
+      } else {
+        f32x2_t bv[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) bv[v] = read_col2(sB[s][0], lane, wn, h, v);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[v][j], av[v], acc[0][j], 0, 0, 0);
+      }
+    }
+  }
+
+  // epilogue: a lane holds row li of the wave's 16 and, as 16-byte pieces, columns
+  // 16 j + 4 g .. + 3 (gate_up, down) or 8 g + 4 j .. + 3 (dgu, dx) of its 32
+  const int lr = 16 * wm + li;
+  if (lr >= nrows) return;
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int64_t o = (row0 + lr) * p.N + n0 + 32 * wn + (kNT ? 16 * j + 4 * g : 8 * g + 4 * j);
+    f32x4_t c;
+    if constexpr (kNT) c = acc[0][j];
+    else c = f32x4_t{acc[0][0][2 * j], acc[0][1][2 * j], acc[0][0][2 * j + 1], acc[0][1][2 * j + 1]};
+    {
+      if constexpr (MODE == kGateUp) {
+        const f32x4_t uu = acc[NB - 1][j];
+        f32x4_t hh;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) hh[v] = silu_f(c[v]) * uu[v];
+        *(f32x4_u*)(p.o0 + o) = c;
+        *(f32x4_u*)(p.o1 + o) = uu;
+        *(f32x4_u*)(p.o2 + o) = hh;
+      } else if constexpr (MODE == kDgu) {
+        const f32x4_t gg = *(const f32x4_u*)(p.g + o), uu = *(const f32x4_u*)(p.u + o);
+        f32x4_t dg, du;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float sig = 1.0f / (1.0f + expf(-gg[v]));
+          du[v] = c[v] * silu_f(gg[v]);                                         // dh * silu(g)
+          dg[v] = (c[v] * uu[v]) * (sig * (1.0f + gg[v] * (1.0f - sig)));       // silu'(g) (dh u)
+        }
+        *(f32x4_u*)(p.o1 + o) = du;
+        *(f32x4_u*)(p.o0 + o) = dg;
+      } else {
+        *(f32x4_u*)(p.o0 + o) = c;
+      }
+    }
+  }
+}
+
+// Weight gradients: out[e][m][n] = sum over expert e's rows r of a[r][m] b[r][n], up to
+// three products per launch (each alone has too few tiles to fill the chip at the sizes
+// this path is used at). Waves: 32 x 32 each.
+struct DwJob {
+  const float* a;  // [R, M]
+  const float* b;  // [R, N]
+  float* out;      // [E, M, N]
+  int M, N;
+};
+struct DwParams {
+  const int64_t* counts;
+  int64_t R;
+  int E;
+  int per_e;  // tiles of one expert, the same in every job: M N / 64^2
+  DwJob job[3];
+};
+
+template <bool ALIGNED>
+__global__ __launch_bounds__(256, 4) void dw_kernel(DwParams p) {
+  __shared__ __attribute__((aligned(1024))) float sA[2][kTile];
+  __shared__ __attribute__((aligned(1024))) float sB[2][kTile];
+  __shared__ int s_tmp[8];
+  __shared__ int s_out[2];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // Workgroup b runs on XCD b % 8. Every XCD takes an eighth of each (job, expert)'s tiles,
+  // neighbouring ones: whole experts per XCD would share more in its L2 but leave XCDs
+  // idle where the experts' row counts differ. The jobs start at experts a third apart:
+  // a CU's workgroups, a chip apart in the grid, would otherwise all belong to the same
+  // heavy expert.
+  const int q = p.per_e % 8 == 0 ? p.per_e >> 3 : 0, b = blockIdx.x;
+  const int group = q ? (b >> 3) / q : b / p.per_e;
+  const int t = q ? (b & 7) * q + (b >> 3) % q : b % p.per_e;
+  const int ji = group / p.E, e = (group + ji * ((p.E + 2) / 3)) % p.E;
+  const DwJob job = ji == 0 ? p.job[0] : (ji == 1 ? p.job[1] : p.job[2]);
+  const int M = job.M, N = job.N, ntn = N / BN;
+  const int m0 = (t / ntn) * BM, n0 = (t % ntn) * BN;
+  Seg seg;
+  find_segment(p.counts, p.R, p.E, e, s_tmp, s_out, seg);
+  const int wm = w >> 1, wn = w & 1, g = lane >> 4, li = lane & 15;
+  const float* A = job.a + (int64_t)seg.start * M + m0;
+  const float* B = job.b + (int64_t)seg.start * N + n0;
+  auto issue = [&](int k0, int s) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int cc = 2 * w + c, k = k0 + krow_of(cc, lane), col = krow_chunk(cc, lane) * 4;
+      const bool in = k < seg.count;
+      copy16<ALIGNED>(in ? A + (int64_t)k * M + col : (const float*)kZeroChunk, lds_addr(sA[s] + cc * 256));
+      copy16<ALIGNED>(in ? B + (int64_t)k * N + col : (const float*)kZeroChunk, lds_addr(sB[s] + cc * 256));
+    }
+  };
+  f32x4_t acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if (seg.count > 0) issue(0, 0);
+  for (int k0 = 0, s = 0; k0 < seg.count; k0 += BK, s ^= 1) {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (k0 + BK < seg.count) issue(k0 + BK, s ^ 1);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      f32x2_t av[4], bv[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        av[j] = read_col2(sA[s], lane, wm, h, j);
+        bv[j] = read_col2(sB[s], lane, wn, h, j);
+      }
+#pragma unroll
+      for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[s4][j], av[s4][i], acc[i][j], 0, 0, 0);
+    }
+  }
+  // m-tile i holds rows 32 wm + 2 li + i; a lane's columns are 32 wn + 8 g .. + 7
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float* o = job.out + ((int64_t)e * M + m0 + 32 * wm + 2 * li + i) * N + n0 + 32 * wn + 8 * g;
+    *(f32x4_u*)o = f32x4_t{acc[i][0][0], acc[i][1][0], acc[i][0][1], acc[i][1][1]};
+    *(f32x4_u*)(o + 4) = f32x4_t{acc[i][0][2], acc[i][1][2], acc[i][0][3], acc[i][1][3]};
+  }
+}
+
+// Zeroes the rows from sum(counts) on of up to four [R, cols] tensors. Almost always there
+// are none and the launch only reads the counts (2 us, where clearing the whole tensors
+// first took 42 us of a 370 us pass at 8192 rows, dim 256, hidden 512).
+struct ZeroParams {
+  const int64_t* counts;
+  int64_t R;
+  int E;
+  float* t[4];
+  int64_t cols[4];
+};
+__global__ __launch_bounds__(256) void zero_rest_kernel(ZeroParams p) {
+  __shared__ int s_tmp[8];
   int cnt[4], st[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -106,209 +402,42 @@ __device__ __forceinline__ void find_segment(const Params& p, int e, int* s_tmp,
     const int64_t c = ee < p.E ? p.counts[ee] : 0;
     cnt[i] = c < 0 ? 0 : (int)(c > p.R ? p.R : c);
   }
-  block_exclusive_scan4(cnt, st, s_tmp);
+  const int64_t total = block_exclusive_scan4(cnt, st, s_tmp);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (threadIdx.x * 4 + i == e) {
-      const int64_t room = p.R - st[i];
-      s_out[0] = st[i];
-      s_out[1] = room <= 0 ? 0 : (cnt[i] > room ? (int)room : cnt[i]);
-    }
-  }
-  __syncthreads();
-  seg.start = s_out[0];
-  seg.count = s_out[1];
-  seg.tile = 0;
-}
-
-// Staging of one 16-k slice.
-//  rows operand [rows, K] (k contiguous), 64 rows: thread t holds row t % 64,
-//    k (t / 64) * 4 .. + 3 (a 16-byte load) and stores them as 4 k-rows.
-//  k-rows operand [k, cols] (cols contiguous), 64 cols: thread t holds k-row
-//    t / 16, cols (t % 16) * 4 .. + 3, stored as one 16-byte LDS write.
-__device__ __forceinline__ float4 load_rows(const float* base, int64_t ld, int row, int nrows, int k) {
-  if (row >= nrows) return make_float4(0.f, 0.f, 0.f, 0.f);
-  return *(const float4*)(base + (int64_t)row * ld + k);
-}
-__device__ __forceinline__ void store_rows(float* tile, const float4& v) {
-  const int r = threadIdx.x & 63, k = (threadIdx.x >> 6) * 4;
-  tile[(k + 0) * LDS_ROW + r] = v.x;
-  tile[(k + 1) * LDS_ROW + r] = v.y;
-  tile[(k + 2) * LDS_ROW + r] = v.z;
-  tile[(k + 3) * LDS_ROW + r] = v.w;
-}
-__device__ __forceinline__ float4 load_krows(const float* base, int64_t ld, int krow, int nk) {
-  if (krow >= nk) return make_float4(0.f, 0.f, 0.f, 0.f);
-  return *(const float4*)(base + (int64_t)krow * ld + (threadIdx.x & 15) * 4);
-}
-__device__ __forceinline__ void store_krows(float* tile, const float4& v) {
-  *(float4*)(tile + (threadIdx.x >> 4) * LDS_ROW + (threadIdx.x & 15) * 4) = v;
-}
-
-// One 16-k slice of MFMAs for this wave's 32 x 32 quarter.
-__device__ __forceinline__ void mma_slice(const float* sa, const float* sb, int wm, int wn, int lane,
-                                          f32x4_t (&acc)[2][2]) {
-#pragma unroll
-  for (int ks = 0; ks < BK; ks += 4) {
-    const int k = ks + (lane >> 4);
-    float av[2], bv[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) av[i] = sa[k * LDS_ROW + 32 * wm + 16 * i + (lane & 15)];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) bv[j] = sb[k * LDS_ROW + 32 * wn + 16 * j + (lane & 15)];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
-  }
-}
-
-// Row-grouped modes: 64 rows of one expert x 64 output columns.
-template <int MODE>
-__global__ __launch_bounds__(256) void rows_kernel(Params p) {
-  constexpr bool kTwoB = MODE == kGateUp;  // two weights into two accumulator sets
-  constexpr bool kNT = MODE == kGateUp || MODE == kDown;  // weights [E, N, K]; else [E, K, N]
-  __shared__ __attribute__((aligned(16))) float sA[BK * LDS_ROW];
-  __shared__ __attribute__((aligned(16))) float sB[BK * LDS_ROW];
-  __shared__ __attribute__((aligned(16))) float sB2[kTwoB ? BK * LDS_ROW : 4];
-  __shared__ int s_tmp[8];
-  __shared__ int s_out[4];
-  int e, mt;
-  Seg seg;
-  find_tile(p, blockIdx.x, s_tmp, s_out, e, seg, mt);
-  if (e < 0) return;
-  const int n0 = blockIdx.y * BN;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 1, wn = w & 1;
-  const int64_t row0 = seg.start + (int64_t)mt * BM;
-  const int nrows = seg.count - mt * BM < BM ? seg.count - mt * BM : BM;
-
-  f32x4_t acc[2][2], acc2[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      acc2[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
-
-  // weight slices for this block: NT [E, N, K] rows n0.. (k contiguous);
-  // NN [E, K, N] k-rows with columns n0..
-  const int phases = MODE == kDx ? 2 : 1;
-  for (int ph = 0; ph < phases; ++ph) {
-    const float* A = (ph == 0 ? p.a : p.a2) + row0 * p.K;
-    const float* Bw = (ph == 0 ? p.b : p.b2) + (int64_t)e * p.N * p.K;
-    const float* B2w = kTwoB ? p.b2 + (int64_t)e * p.N * p.K : nullptr;
-    const int ar = threadIdx.x & 63, ak = (threadIdx.x >> 6) * 4;
-    float4 ra, rb, rb2;
-    auto fetch = [&](int k0) {
-      ra = load_rows(A, p.K, ar, nrows, k0 + ak);
-      if (kNT) {
-        rb = load_rows(Bw + (int64_t)n0 * p.K, p.K, ar, BN, k0 + ak);
-        if (kTwoB) rb2 = load_rows(B2w + (int64_t)n0 * p.K, p.K, ar, BN, k0 + ak);
-      } else {
-        rb = load_krows(Bw + (int64_t)k0 * p.N + n0, p.N, threadIdx.x >> 4, BK);
-      }
-    };
-    fetch(0);
-    for (int k0 = 0; k0 < p.K; k0 += BK) {
-      __syncthreads();  // the previous slice's reads are done
-      store_rows(sA, ra);
-      if (kNT) {
-        store_rows(sB, rb);
-        if (kTwoB) store_rows(sB2, rb2);
-      } else {
-        store_krows(sB, rb);
-      }
-      __syncthreads();
-      if (k0 + BK < p.K) fetch(k0 + BK);
-      mma_slice(sA, sB, wm, wn, lane, acc);
-      if (kTwoB) mma_slice(sA, sB2, wm, wn, lane, acc2);
-    }
-  }
-
-  // epilogue: lane holds rows 4 (lane / 16) + v of each 16 x 16 tile, column lane % 16
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int lr = 32 * wm + 16 * i + 4 * (lane >> 4) + v;
-        if (lr >= nrows) continue;
-        const int64_t r = row0 + lr;
-        const int64_t o = r * p.N + n0 + 32 * wn + 16 * j + (lane & 15);
-        const float c = acc[i][j][v];
-        if (MODE == kGateUp) {
-          const float uu = acc2[i][j][v];
-          p.o0[o] = c;
-          p.o1[o] = uu;
-          p.o2[o] = silu_f(c) * uu;
-        } else if (MODE == kDgu) {
-          const float gg = p.g[o], uu = p.u[o];
-          const float sig = 1.0f / (1.0f + expf(-gg));
-          p.o1[o] = c * silu_f(gg);                               // du = dh * silu(g)
-          p.o0[o] = (c * uu) * (sig * (1.0f + gg * (1.0f - sig)));  // dg = silu'(g) (dh u)
-        } else {
-          p.o0[o] = c;
-        }
-      }
-}
-
-// Weight gradients: out[e][m][n] = sum over expert e's rows r of a[r][m] b[r][n].
-__global__ __launch_bounds__(256) void dw_kernel(Params p) {
-  __shared__ __attribute__((aligned(16))) float sA[BK * LDS_ROW];
-  __shared__ __attribute__((aligned(16))) float sB[BK * LDS_ROW];
-  __shared__ int s_tmp[8];
-  __shared__ int s_out[2];
-  const int e = blockIdx.x;
-  Seg seg;
-  find_segment(p, e, s_tmp, s_out, seg);
-  const int M = p.K, N = p.N;
-  const int ntn = N / BN;
-  const int m0 = (blockIdx.y / ntn) * BM, n0 = (blockIdx.y % ntn) * BN;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 1, wn = w & 1;
-  f32x4_t acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const float* A = p.a + seg.start * M + m0;
-  const float* B = p.b + seg.start * N + n0;
-  float4 ra, rb;
-  auto fetch = [&](int k0) {
-    ra = load_krows(A + (int64_t)k0 * M, M, threadIdx.x >> 4, seg.count - k0);
-    rb = load_krows(B + (int64_t)k0 * N, N, threadIdx.x >> 4, seg.count - k0);
-  };
-  if (seg.count > 0) fetch(0);
-  for (int k0 = 0; k0 < seg.count; k0 += BK) {
-    __syncthreads();
-    store_krows(sA, ra);
-    store_krows(sB, rb);
-    __syncthreads();
-    if (k0 + BK < seg.count) fetch(k0 + BK);
-    mma_slice(sA, sB, wm, wn, lane, acc);
-  }
-  float* out = p.o0 + (int64_t)e * M * N;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int m = m0 + 32 * wm + 16 * i + 4 * (lane >> 4) + v;
-        out[(int64_t)m * N + n0 + 32 * wn + 16 * j + (lane & 15)] = acc[i][j][v];
-      }
+  for (int q = 0; q < 4; ++q)
+    for (int64_t i = total * p.cols[q] + (int64_t)blockIdx.x * 256 + threadIdx.x; i < p.R * p.cols[q];
+         i += (int64_t)gridDim.x * 256)
+      p.t[q][i] = 0.f;
 }
 
 inline bool dims_ok(int64_t R, int E, int a, int b) {
   return R >= 0 && E >= 1 && E <= kMaxE && a >= 64 && b >= 64 && a % 64 == 0 && b % 64 == 0;
 }
 
+inline bool aligned16(const void* a, const void* b, const void* c, const void* d) {
+  return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d) & 15) == 0;
+}
+
 template <int MODE>
 int launch_rows(const Params& p, hipStream_t stream) {
   if (p.R == 0) return kOk;
-  const int64_t gx = (p.R + BM - 1) / BM + p.E;  // >= sum over experts of ceil(count / 64)
-  hipLaunchKernelGGL(rows_kernel<MODE>, dim3((unsigned)gx, (unsigned)(p.N / BN)), dim3(256), 0, stream, p);
+  // >= sum over experts of ceil(count / 64), and as many more as 64-row tiles past the segments
+  const int64_t gx = (p.R + BM - 1) / BM + p.E, grid = gx * (p.N / BN);
+  if (grid > 0x7fffffff) return kErrUnsupportedShape;
+  const dim3 blocks((unsigned)grid), threads(512);
+  if (aligned16(p.a, p.a2, p.b, p.b2)) hipLaunchKernelGGL((rows_kernel<MODE, true>), blocks, threads, 0, stream, p);
+  else hipLaunchKernelGGL((rows_kernel<MODE, false>), blocks, threads, 0, stream, p);
+  return launch_status();
+}
+
+int launch_dw(DwParams& p, int jobs, hipStream_t stream) {
+  const int64_t per_e = (int64_t)(p.job[0].M / BM) * (p.job[0].N / BN), grid = per_e * p.E * jobs;
+  if (grid > 0x7fffffff) return kErrUnsupportedShape;
+  p.per_e = (int)per_e;
+  bool aligned = true;
+  for (int j = 0; j < jobs; ++j) aligned = aligned && aligned16(p.job[j].a, p.job[j].b, nullptr, nullptr);
+  if (aligned) hipLaunchKernelGGL(dw_kernel<true>, dim3((unsigned)grid), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL(dw_kernel<false>, dim3((unsigned)grid), dim3(256), 0, stream, p);
   return launch_status();
 }
 
@@ -365,10 +494,34 @@ MOE_API int moe_grouped_gemm_f32_bwd_dw(const float* a, const float* b, const in
                                         int32_t n_experts, int32_t m, int32_t n, float* out, hipStream_t stream) {
   if (!dims_ok(n_rows, n_experts, m, n)) return kErrInvalidArgument;
   if (!counts || !out || (n_rows > 0 && (!a || !b))) return kErrInvalidArgument;
-  Params p{};
-  p.counts = counts; p.R = n_rows; p.E = n_experts; p.N = n; p.K = m;
-  p.a = a; p.b = b; p.o0 = out;
-  const int64_t tiles = (int64_t)(m / BM) * (n / BN);
-  hipLaunchKernelGGL(dw_kernel, dim3((unsigned)n_experts, (unsigned)tiles), dim3(256), 0, stream, p);
+  DwParams p{};
+  p.counts = counts; p.R = n_rows; p.E = n_experts;
+  p.job[0] = DwJob{a, b, out, m, n};
+  return launch_dw(p, 1, stream);
+}
+
+MOE_API int moe_grouped_gemm_f32_bwd_dw_all(const float* dg, const float* du, const float* dy, const float* x,
+                                            const float* h, const int64_t* counts, int64_t n_rows, int32_t n_experts,
+                                            int32_t dim, int32_t hidden, float* dw1, float* dw3, float* dw2,
+                                            hipStream_t stream) {
+  if (!dims_ok(n_rows, n_experts, dim, hidden)) return kErrInvalidArgument;
+  if (!counts || !dw1 || !dw2 || !dw3 || (n_rows > 0 && (!dg || !du || !dy || !x || !h))) return kErrInvalidArgument;
+  DwParams p{};
+  p.counts = counts; p.R = n_rows; p.E = n_experts;
+  p.job[0] = DwJob{dg, x, dw1, hidden, dim};
+  p.job[1] = DwJob{du, x, dw3, hidden, dim};
+  p.job[2] = DwJob{dy, h, dw2, dim, hidden};
+  return launch_dw(p, 3, stream);
+}
+
+MOE_API int moe_zero_rows_past_f32(const int64_t* counts, int64_t n_rows, int32_t n_experts, float* t0, int64_t cols0,
+                                   float* t1, int64_t cols1, float* t2, int64_t cols2, float* t3, int64_t cols3,
+                                   hipStream_t stream) {
+  if (n_rows < 0 || n_experts < 1 || n_experts > kMaxE || !counts) return kErrInvalidArgument;
+  if (cols0 < 0 || cols1 < 0 || cols2 < 0 || cols3 < 0) return kErrInvalidArgument;
+  if ((cols0 && !t0) || (cols1 && !t1) || (cols2 && !t2) || (cols3 && !t3)) return kErrInvalidArgument;
+  if (n_rows == 0) return kOk;
+  const ZeroParams p{counts, n_rows, n_experts, {t0, t1, t2, t3}, {cols0, cols1, cols2, cols3}};
+  hipLaunchKernelGGL(zero_rest_kernel, dim3(64), dim3(256), 0, stream, p);
   return launch_status();
 }

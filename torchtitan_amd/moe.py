@@ -56,7 +56,7 @@ def _run_experts_for_loop(
     product rounded to bf16) are those of the reference's bf16 matmuls. As in the
     reference, reading sum(counts) synchronises with the host."""
     total = int(num_tokens_per_expert.sum().item())
-    xs = x[:total]
+    xs = x if total == x.shape[0] else x[:total]  # a slice's backward copies the gradient
     if x.dtype == torch.float32:
         if not (w1.dtype == w2.dtype == w3.dtype == torch.float32):
             raise TypeError(f"expected float32 expert weights for float32 x, got {w1.dtype}, {w2.dtype}, {w3.dtype}")

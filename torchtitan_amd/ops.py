@@ -469,11 +469,12 @@ def grouped_swiglu_f32(
     counts = num_tokens_per_expert.to(torch.int64).contiguous()
     r, d = x.shape
     e, h_dim, _ = w1.shape
-    g = x.new_zeros(r, h_dim)
-    u = x.new_zeros(r, h_dim)
-    h = x.new_zeros(r, h_dim)
-    y = x.new_zeros(r, d)
+    g = x.new_empty(r, h_dim)
+    u = x.new_empty(r, h_dim)
+    h = x.new_empty(r, h_dim)
+    y = x.new_empty(r, d)
     s = stream_of(x)
+    call("moe_zero_rows_past_f32", ptr(counts), r, e, ptr(g), h_dim, ptr(u), h_dim, ptr(h), h_dim, ptr(y), d, s)
     call("moe_grouped_gemm_f32_gate_up", ptr(x), ptr(w1), ptr(w3), ptr(counts), r, e, d, h_dim,
          ptr(g), ptr(u), ptr(h), s)
     call("moe_grouped_gemm_f32_down", ptr(h), ptr(w2), ptr(counts), r, e, d, h_dim, ptr(y), s)
@@ -497,20 +498,20 @@ def grouped_swiglu_f32_backward(
     counts = num_tokens_per_expert.to(torch.int64).contiguous()
     r, d = x.shape
     e, h_dim, _ = w1.shape
-    dg = x.new_zeros(r, h_dim)
-    du = x.new_zeros(r, h_dim)
-    dx = x.new_zeros(r, d)
+    dg = x.new_empty(r, h_dim)
+    du = x.new_empty(r, h_dim)
+    dx = x.new_empty(r, d)
     dw1 = torch.empty_like(w1)
     dw2 = torch.empty_like(w2)
     dw3 = torch.empty_like(w3)
     s = stream_of(x)
+    call("moe_zero_rows_past_f32", ptr(counts), r, e, ptr(dg), h_dim, ptr(du), h_dim, ptr(dx), d, None, 0, s)
     call("moe_grouped_gemm_f32_bwd_dgu", ptr(dy), ptr(w2), ptr(g), ptr(u), ptr(counts), r, e, d, h_dim,
          ptr(dg), ptr(du), s)
     call("moe_grouped_gemm_f32_bwd_dx", ptr(dg), ptr(du), ptr(w1), ptr(w3), ptr(counts), r, e, d, h_dim,
          ptr(dx), s)
-    call("moe_grouped_gemm_f32_bwd_dw", ptr(dg), ptr(x), ptr(counts), r, e, h_dim, d, ptr(dw1), s)
-    call("moe_grouped_gemm_f32_bwd_dw", ptr(du), ptr(x), ptr(counts), r, e, h_dim, d, ptr(dw3), s)
-    call("moe_grouped_gemm_f32_bwd_dw", ptr(dy), ptr(h), ptr(counts), r, e, d, h_dim, ptr(dw2), s)
+    call("moe_grouped_gemm_f32_bwd_dw_all", ptr(dg), ptr(du), ptr(dy), ptr(x), ptr(h), ptr(counts), r, e, d, h_dim,
+         ptr(dw1), ptr(dw3), ptr(dw2), s)
     return dx, dw1, dw2, dw3
 
 
