@@ -1,0 +1,108 @@
+"""The transposing quantizers that run a block per 128 rows, at the edges of those chunks
+(groups of 0, 1, 127 to 129 and several hundred rows, one group, more groups than a wave
+scans, rows and columns past the last group), byte for byte against the quantizers that
+work another way: the MX row quantizer on each group transposed and zero padded in torch,
+and the fp8 ones that take their own amax in a pass over a whole group.
+"""
+
+import pytest
+import torch
+
+from tests.conftest import banner
+
+pytestmark = pytest.mark.gpu
+
+CASES = {  # rows of each group, rows past them, columns
+    "edges": ([127, 128, 129, 0, 1, 0, 300], 0, 128),
+    "one_group": ([130], 5, 64),
+    "last_empty": ([5, 257, 0], 40, 192),
+    "many_groups": ([(37 * i) % 141 for i in range(257)], 9, 64),
+    "wave_of_groups": ([(53 * i) % 150 for i in range(256)], 0, 128),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_token_chunks(dev, name):
+    from torchtitan_amd import _lib
+    from torchtitan_amd._lib import call, ptr
+
+    groups, rest, c = CASES[name]
+    banner(f"token quantizers by chunks {name}")
+    e, r = len(groups), sum(groups) + rest
+    gen = torch.Generator(device=dev).manual_seed(5)
+    x = (torch.randn(r, c, generator=gen, device=dev) * torch.randn(r, 1, generator=gen, device=dev).exp()).bfloat16()
+    counts = torch.tensor(groups, dtype=torch.int64, device=dev)
+    rpad = (int(_lib.lib().moe_mxfp8_padded_rows(r, e)) + 127) // 128 * 128
+    st = torch.cuda.current_stream().cuda_stream
+
+    def u8(*shape):
+        return torch.full(shape, 0xA5, dtype=torch.uint8, device=dev)
+
+    qr, sr, qt, s = u8(r, c), u8(r, c // 32), u8(c, rpad), u8(rpad // 32, c)
+    call("moe_mxfp8_quant_dual_tokens", ptr(x), ptr(counts), r, e, c, rpad, ptr(qr), ptr(sr), ptr(qt), ptr(s), st)
+    wr, ws = u8(r, c), u8(r, c // 32)
+    call("moe_mxfp8_quant_rows", ptr(x), r, c, ptr(wr), ptr(ws), st)
+    n = sum(groups)
+    assert torch.equal(qr[:n], wr[:n]) and torch.equal(sr[:n], ws[:n])
+    want_q, want_s = torch.zeros_like(qt), torch.zeros_like(s)
+    start = pstart = 0
+    for g in groups:
+        pad = (g + 127) // 128 * 128
+        if g:
+            t = torch.zeros(c, pad, dtype=torch.bfloat16, device=dev)
+            t[:, :g] = x[start:start + g].t()
+            q1, s1 = u8(c, pad), u8(c, pad // 32)
+            call("moe_mxfp8_quant_rows", ptr(t), c, pad, ptr(q1), ptr(s1), st)
+            want_q[:, pstart:pstart + pad] = q1
+            want_s[pstart // 32:(pstart + pad) // 32] = s1.t()
+        start, pstart = start + g, pstart + pad
+    assert torch.equal(qt, want_q) and torch.equal(s, want_s)
+
+    # fp8: from the groups' known amax, and with its own amax pass
+    amax = torch.zeros(e, c, device=dev)
+    start = 0
+    for i, g in enumerate(groups):
+        if g:
+            amax[i] = x[start:start + g].float().abs().amax(0)
+        start += g
+    outs = []
+    for known in (True, False):
+        q, sc = u8(c, rpad), torch.zeros(e, c, device=dev)
+        if known:
+            call("moe_fp8_quant_tokens_t_amax", ptr(x), ptr(amax), ptr(counts), r, e, c, rpad, ptr(q), ptr(sc), st)
+        else:
+            call("moe_fp8_quant_tokens_t", ptr(x), ptr(counts), r, e, c, rpad, ptr(q), ptr(sc), st)
+        outs.append((q, sc))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("a,b", [(32, 64), (128, 128), (160, 192), (352, 128)])
+def test_weight_chunks(dev, a, b):
+    from torchtitan_amd._lib import call, ptr
+
+    banner(f"weight quantizers by chunks {a} x {b}")
+    e = 3
+    gen = torch.Generator(device=dev).manual_seed(6)
+    x = (torch.randn(e, a, b, generator=gen, device=dev) * torch.randn(e, 1, b, generator=gen, device=dev).exp()).bfloat16()
+    st = torch.cuda.current_stream().cuda_stream
+
+    def u8(*shape):
+        return torch.full(shape, 0xA5, dtype=torch.uint8, device=dev)
+
+    q, s, qt, t = u8(e, a, b), u8(e, a, b // 32), u8(e, b, a), u8(e, b, a // 32)
+    call("moe_mxfp8_quant_dual_cols", ptr(x), e, a, b, ptr(q), ptr(s), ptr(qt), a * b, a, ptr(t), b * (a // 32),
+         a // 32, st)
+    wq, ws, wqt, wt = u8(e, a, b), u8(e, a, b // 32), u8(e, b, a), u8(e, b, a // 32)
+    xt = x.transpose(1, 2).contiguous()
+    call("moe_mxfp8_quant_rows", ptr(x), e * a, b, ptr(wq), ptr(ws), st)
+    call("moe_mxfp8_quant_rows", ptr(xt), e * b, a, ptr(wqt), ptr(wt), st)
+    for got, want in ((q, wq), (s, ws), (qt, wqt), (t, wt)):
+        assert torch.equal(got, want)
+    q2, t2 = u8(e, b, a), u8(e, b, a // 32)
+    call("moe_mxfp8_quant_cols_t", ptr(x), e, a, b, ptr(q2), a * b, a, ptr(t2), b * (a // 32), a // 32, st)
+    assert torch.equal(q2, wqt) and torch.equal(t2, wt)
+    amax = x.float().abs().amax(1).contiguous()
+    f = [(u8(e, b, a), torch.zeros(e, b, device=dev)) for _ in range(2)]
+    call("moe_fp8_quant_cols_t_amax", ptr(x), ptr(amax), e, a, b, ptr(f[0][0]), a * b, a, ptr(f[0][1]), b, st)
+    call("moe_fp8_quant_cols_t", ptr(x), e, a, b, ptr(f[1][0]), a * b, a, ptr(f[1][1]), b, st)
+    assert torch.equal(f[0][0], f[1][0]) and torch.equal(f[0][1], f[1][1])

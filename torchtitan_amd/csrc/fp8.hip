@@ -468,19 +468,30 @@ constexpr int kTRows = 128;  // slab rows transposed per pass
 // of 16 rows of one column (2-byte reads; the swizzle keeps the eight row
 // groups a wave reads at once in distinct banks) and stores their 16 bytes, so
 // that 8 consecutive lanes write 128 contiguous bytes of one output row. The
-// loads two passes ahead are issued as soon as the tile is in LDS. 128-column
+// loads two passes ahead are issued as soon as the tile is in LDS.
+// ONE: the slab is a single pass of at most 128 rows. Nothing is loaded ahead, so a
+// thread needs half the registers (107-116 -> 55 VGPRs) and four blocks share a CU
+// instead of two, and a launch has blocks for every 128 rows: the other blocks, and not
+// this block's own passes, keep loads and stores in flight, and no block outlasts the
+// rest where groups differ or one more round of blocks is nearly empty. us, a block per
+// slab and group or expert, and per 128 rows: MX dual tokens 64 groups, 32768 x 2304 116
+// -> 75 (2.6 -> 4.0 TB/s), x 1024 52 -> 32, 256 groups, 131072 x 2304 385 -> 292; MX dual
+// cols 64 x 1024 x 2304 150 -> 119 (5.1 TB/s), 64 x 2304 x 1024 150 -> 122; fp8 tokens 49
+// -> 41 (5.5 TB/s), 26 -> 21; fp8 cols 96 -> 82, 98 -> 78 (5.8 TB/s); 16 groups, 4096 x
+// 2304 25 -> 16 and 15 -> 10. Only the fp8 quantizers that first take their own amax keep
+// the passes. 128-column
 // slabs (launched whenever the width allows) write the row-wise layout in whole
 // 128-byte lines: 2-12 % faster than 64-column ones at the Kimi shapes.
 // GATHER: the slab's rows are gathered (RowGather); the indices are loaded two
 // passes ahead of the rows they address and the scale is applied when a pass is
 // consumed, so neither waits behind the row loads in flight.
-template <bool MX, bool ROWS, int COLS, bool GATHER = false>
+template <bool MX, bool ROWS, int COLS, bool GATHER = false, bool ONE = false>
 __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, int64_t ld, int n_rows, int n_out,
                                              uint8_t* __restrict__ out, int64_t ldo, uint8_t* __restrict__ sc,
                                              int64_t sc_b, int64_t sc_k, const float* s_col, uint32_t* s_tile,
                                              uint8_t* __restrict__ qr = nullptr, int64_t ldr = 0,
                                              uint8_t* __restrict__ sr = nullptr, int64_t ldsr = 0,
-                                             RowGather gather = RowGather{}, int shift = 0) {
+                                             RowGather gather = RowGather{}) {
   constexpr int T = 4 * COLS, CPR = COLS / 8;
   const int t = threadIdx.x;
   auto in_rows = [&](int row) { return row >= 0 && row < n_rows; };
@@ -578,8 +589,10 @@ __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, 
 #pragma unroll
     for (int w = 0; w < T / 64; ++w) any_nan |= s_wnan[w];
     const bool fast = any_nan == 0u;  // block-uniform: the tile holds no NaN
-    load(v, ix, sv, ok, a0 + 2 * kTRows);
-    if constexpr (GATHER) load_idx(ix, a0 + 4 * kTRows);
+    if constexpr (!ONE) {
+      load(v, ix, sv, ok, a0 + 2 * kTRows);
+      if constexpr (GATHER) load_idx(ix, a0 + 4 * kTRows);
+    }
     // unit (column cc, rows 16 kq .. 16 kq + 15 of the pass): 8 consecutive lanes cover one
     // output row's 128 bytes, so every store instruction writes 8 rows x 128 contiguous bytes
 #pragma unroll
@@ -624,76 +637,148 @@ __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, 
       }
     }
   };
-  // passes start `shift` rows before the slab (rows < 0 are neither loaded nor
-  // stored), so that with shift = the output offset mod 128 every pass writes
-  // whole 128-byte lines of each output row
-  const int b0 = -shift;
-  if constexpr (GATHER) {
-    load_idx(ia, b0);
-    load_idx(ib, b0 + kTRows);
-  }
   uint32_t oka, okb;
-  load(va, ia, sa, oka, b0);
-  if constexpr (GATHER) load_idx(ia, b0 + 2 * kTRows);
-  load(vb, ib, sb, okb, b0 + kTRows);
-  if constexpr (GATHER) load_idx(ib, b0 + 3 * kTRows);
-  for (int a0 = b0; a0 < n_out; a0 += 2 * kTRows) {
+  if constexpr (ONE) {
+    if constexpr (GATHER) load_idx(ia, 0);
+    load(va, ia, sa, oka, 0);
+    pass(va, ia, sa, oka, 0);
+    return;
+  }
+  if constexpr (GATHER) {
+    load_idx(ia, 0);
+    load_idx(ib, kTRows);
+  }
+  load(va, ia, sa, oka, 0);
+  if constexpr (GATHER) load_idx(ia, 2 * kTRows);
+  load(vb, ib, sb, okb, kTRows);
+  if constexpr (GATHER) load_idx(ib, 3 * kTRows);
+  for (int a0 = 0; a0 < n_out; a0 += 2 * kTRows) {
     pass(va, ia, sa, oka, a0);
     if (a0 + kTRows < n_out) pass(vb, ib, sb, okb, a0 + kTRows);
   }
 }
 
 // x [E][A][B] -> q rows (e, b) of A values at q + e * q_estride + b * q_ld, and
-// scale[e * s_estride + b] = amax over A. Block per (e, COLS columns). With
-// amax_in (the column amax [E][B] already known, from quant_rows_colamax_kernel)
-// the amax pass is skipped and x is read once.
-template <int COLS>
+// scale[e * s_estride + b] = amax over A. With amax_in (the column amax [E][B] already
+// known, from quant_rows_colamax_kernel) x is read once, by a block per (e, COLS columns,
+// 128 rows) (ONE); else a block per (e, COLS columns) takes the amax in a pass of its own.
+template <int COLS, bool ONE>
 __global__ __launch_bounds__(4 * COLS) void quant_cols_t_kernel(const uint16_t* __restrict__ x, int A, int B,
                                                            uint8_t* __restrict__ q, int64_t q_estride, int64_t q_ld,
                                                            float* __restrict__ scale, int64_t s_estride,
                                                            const float* __restrict__ amax_in) {
-  __shared__ float s_red[COLS * 33];
+  __shared__ float s_red[ONE ? 1 : COLS * 33];
   __shared__ float s_amax[COLS];
   __shared__ __attribute__((aligned(16))) uint32_t s_tile[kTRows * (COLS / 2)];
-  const int nb = B / COLS;
-  const int64_t e = blockIdx.x / nb;
-  const int b0 = (blockIdx.x % nb) * COLS;
+  const int nb = B / COLS, nch = ONE ? (A + kTRows - 1) / kTRows : 1;
+  const int64_t e = blockIdx.x / (nb * nch);
+  const int b0 = (blockIdx.x / nch % nb) * COLS, a0 = blockIdx.x % nch * kTRows;
   const uint16_t* base = x + e * A * (int64_t)B + b0;
-  if (amax_in) {
+  if constexpr (ONE) {
     if (threadIdx.x < COLS) s_amax[threadIdx.x] = amax_in[e * B + b0 + threadIdx.x];
-    __syncthreads();
   } else {
     slab_amax<COLS>(base, B, A, s_red, s_amax);
   }
-  if (threadIdx.x < COLS) {
+  if (threadIdx.x < COLS) {  // (its own column's amax)
     const float s = scale_of(s_amax[threadIdx.x]);
     s_amax[threadIdx.x] = s;
-    scale[e * s_estride + b0 + threadIdx.x] = s;
+    if (a0 == 0) scale[e * s_estride + b0 + threadIdx.x] = s;
   }
   __syncthreads();
-  slab_t_quant<false, false, COLS>(base, B, A, A, q + e * q_estride + b0 * q_ld, q_ld, nullptr, 0, 0, s_amax, s_tile);
+  const int n = ONE ? min(kTRows, A - a0) : A;
+  slab_t_quant<false, false, COLS, false, ONE>(base + (int64_t)a0 * B, B, n, n, q + e * q_estride + b0 * q_ld + a0, q_ld, nullptr, 0,
+                                   0, s_amax, s_tile);
+}
+
+// The 128 rows of one token group that a block transposes: rows off .. of group e, which
+// starts at row seg0 and at pstart of the padded layout (its 128-row chunks before it times
+// 128) and has n rows. Past the last chunk e is -1, off counts the chunks past it and seg0,
+// pstart, n describe the last group. Every thread of the block calls it. Up to 256 groups
+// every wave scans the counts by itself, without barriers: a block moves one 128-row tile,
+// and three block-wide scans before it took as long as the tile.
+constexpr int kTailBlocks = 8;  // per slab, for the columns past the last group
+struct GroupChunk { int e, seg0, pstart, n, off; };
+__device__ __forceinline__ GroupChunk find_chunk(const int64_t* __restrict__ counts, int64_t R, int E, int ci,
+                                                 int* s_tmp, GroupChunk* s_out) {
+  static_assert(kPad == 128 && kMxPad == 128, "a group's padding is whole chunks");
+  const bool small = E <= 256;
+  const int t = small ? (threadIdx.x & 63) : threadIdx.x;
+  int cnt[4], ch[4], st[4], cst[4], total;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int ee = t * 4 + i;
+    const int64_t c = ee < E ? counts[ee] : 0;
+    cnt[i] = c < 0 ? 0 : (int)(c > R ? R : c);
+    ch[i] = cnt[i] / kTRows + (cnt[i] % kTRows != 0);
+  }
+  if (small) {
+    int a = cnt[0] + cnt[1] + cnt[2] + cnt[3], b = ch[0] + ch[1] + ch[2] + ch[3];
+    const int la = a, lb = b;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int oa = __shfl_up(a, off), ob = __shfl_up(b, off);
+      if (t >= off) { a += oa; b += ob; }
+    }
+    total = __builtin_amdgcn_readlane(b, 63);
+    int ra = a - la, rb = b - lb;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      st[i] = ra; ra += cnt[i];
+      cst[i] = rb; rb += ch[i];
+    }
+  } else {
+    block_exclusive_scan4(cnt, st, s_tmp);
+    total = block_exclusive_scan4(ch, cst, s_tmp);
+  }
+  GroupChunk g{-1, 0, 0, 0, 0};
+  bool found = false;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int ee = t * 4 + i;
+    const bool mine = ee < E && ci >= cst[i] && ci < cst[i] + ch[i];
+    if (mine || (ci >= total && ee == E - 1)) {
+      g = GroupChunk{mine ? ee : -1, st[i], cst[i] * kTRows, cnt[i], mine ? (ci - cst[i]) * kTRows : ci - total};
+      found = true;
+    }
+  }
+  if (small) {
+    const int l = (int)__builtin_ctzll(__ballot(found));
+    return GroupChunk{__builtin_amdgcn_readlane(g.e, l), __builtin_amdgcn_readlane(g.seg0, l),
+                      __builtin_amdgcn_readlane(g.pstart, l), __builtin_amdgcn_readlane(g.n, l),
+                      __builtin_amdgcn_readlane(g.off, l)};
+  }
+  if (found) *s_out = g;
+  __syncthreads();
+  return *s_out;
 }
 
 // x [R][C] with expert token groups (counts) -> q [C][Rpad] (group e at the
 // 128-aligned offset pstart_e, zero padded to ceil128(count_e)), scale [E][C].
-// Block per (e, COLS columns); empty groups exit. With amax_in (the column amax
-// [E][C] of every group already known, from quant_rows_groupamax_kernel) the
-// amax pass is skipped and x is read once.
-template <int COLS, bool GATHER = false>
+// With amax_in (the column amax [E][C] of every group already known, from
+// quant_rows_groupamax_kernel) x is read once, by a block per (128 rows of a group, COLS
+// columns) (ONE); else a block per (e, COLS columns) takes the amax in a pass of its own.
+template <int COLS, bool ONE, bool GATHER = false>
 __global__ __launch_bounds__(4 * COLS) void quant_tokens_t_kernel(const uint16_t* __restrict__ x, const int64_t* __restrict__ counts,
                                                              int64_t R, int E, int C, int64_t Rpad,
                                                              uint8_t* __restrict__ q, float* __restrict__ scale,
                                                              const float* __restrict__ amax_in, RowGather gather) {
-  __shared__ float s_red[COLS * 33];
+  static_assert(ONE || !GATHER, "a gathered operand comes with its amax");
+  __shared__ float s_red[ONE ? 1 : COLS * 33];
   __shared__ float s_amax[COLS];
   __shared__ __attribute__((aligned(16))) uint32_t s_tile[kTRows * (COLS / 2)];
   __shared__ int s_tmp[8];
   __shared__ int s_seg[2];
+  __shared__ GroupChunk s_gc;
   // slab-major: the blocks running together share column slabs (1-4 % faster
   // than expert-major at the Kimi shapes)
-  const int e = blockIdx.x % E;
-  const int c0 = (blockIdx.x / E) * COLS;
-  {
+  const int n_chunks = ONE ? (int)(R / kTRows) + E : E;
+  const int c0 = (blockIdx.x / n_chunks) * COLS;
+  int e = blockIdx.x % n_chunks, seg0, pstart, n, off = 0;
+  if constexpr (ONE) {
+    const GroupChunk gc = find_chunk(counts, R, E, e, s_tmp, &s_gc);
+    if (gc.e < 0) return;
+    e = gc.e; seg0 = gc.seg0; pstart = gc.pstart; n = gc.n; off = gc.off;
+  } else {
     int cnt[4], pc[4], st[4], pst[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -706,35 +791,34 @@ __global__ __launch_bounds__(4 * COLS) void quant_tokens_t_kernel(const uint16_t
     block_exclusive_scan4(pc, pst, s_tmp);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (threadIdx.x * 4 + i == e) { s_seg[0] = st[i]; s_seg[1] = pst[i]; s_red[0] = __int_as_float(cnt[i]); }
+      if (threadIdx.x * 4 + i == e) s_gc = GroupChunk{e, st[i], pst[i], cnt[i], 0};
     __syncthreads();
+    seg0 = s_gc.seg0; pstart = s_gc.pstart; n = s_gc.n;
   }
-  const int seg0 = s_seg[0], pstart = s_seg[1];
-  int n = __float_as_int(s_red[0]);
-  __syncthreads();
   if ((int64_t)seg0 + n > R) n = (int)(R - seg0 > 0 ? R - seg0 : 0);
   const int n_out = (n + kPad - 1) / kPad * kPad;
-  if (n == 0 || (int64_t)pstart + n_out > Rpad) return;
-  const uint16_t* base = GATHER ? nullptr : x + (int64_t)seg0 * C + c0;
+  if (n <= off || (int64_t)pstart + n_out > Rpad) return;
+  const int64_t r0 = (int64_t)seg0 + off;
+  const uint16_t* base = GATHER ? nullptr : x + r0 * C + c0;
   if constexpr (GATHER) {  // this slab's rows and columns of the gathered source
     gather.src += c0;
-    gather.idx += seg0;
-    if (gather.scale) gather.scale += seg0;
+    gather.idx += r0;
+    if (gather.scale) gather.scale += r0;
   }
-  if (GATHER || amax_in) {  // a gathered operand comes with its amax
+  if constexpr (ONE) {
     if (threadIdx.x < COLS) s_amax[threadIdx.x] = amax_in[(int64_t)e * C + c0 + threadIdx.x];
-    __syncthreads();
   } else {
     slab_amax<COLS>(base, C, n, s_red, s_amax);
   }
-  if (threadIdx.x < COLS) {
+  if (threadIdx.x < COLS) {  // (its own column's amax)
     const float s = scale_of(s_amax[threadIdx.x]);
     s_amax[threadIdx.x] = s;
-    scale[(int64_t)e * C + c0 + threadIdx.x] = s;
+    if (off == 0) scale[(int64_t)e * C + c0 + threadIdx.x] = s;
   }
   __syncthreads();
-  slab_t_quant<false, false, COLS, GATHER>(base, C, n, n_out, q + (int64_t)c0 * Rpad + pstart, Rpad, nullptr, 0, 0,
-                                           s_amax, s_tile, nullptr, 0, nullptr, 0, gather, pstart % 128);
+  slab_t_quant<false, false, COLS, GATHER, ONE>(base, C, ONE ? min(n - off, kTRows) : n, ONE ? kTRows : n_out,
+                                                q + (int64_t)c0 * Rpad + pstart + off, Rpad, nullptr, 0, 0, s_amax,
+                                                s_tile, nullptr, 0, nullptr, 0, gather);
 }
 
 // ---------------------------------------------------------------------------
@@ -773,41 +857,41 @@ __global__ __launch_bounds__(256) void mx_quant_rows_kernel(const uint4* __restr
 }
 
 // x [E][A][B] -> q rows (e, b) of A values at q + e * q_estride + b * q_ld, and
-// their A/32 scales at s + e * s_estride + b * s_ld. Block per (e, COLS columns).
+// their A/32 scales at s + e * s_estride + b * s_ld. Block per (e, COLS columns, 128 rows).
 template <int COLS>
 __global__ __launch_bounds__(4 * COLS) void mx_quant_cols_t_kernel(const uint16_t* __restrict__ x, int A, int B,
                                                               uint8_t* __restrict__ q, int64_t q_estride,
                                                               int64_t q_ld, uint8_t* __restrict__ s,
                                                               int64_t s_estride, int64_t s_ld) {
   __shared__ __attribute__((aligned(16))) uint32_t s_tile[kTRows * (COLS / 2)];
-  const int nb = B / COLS;
-  const int64_t e = blockIdx.x / nb;
-  const int b0 = (blockIdx.x % nb) * COLS;
-  slab_t_quant<true, false, COLS>(x + e * A * (int64_t)B + b0, B, A, A, q + e * q_estride + b0 * q_ld, q_ld,
-                            s + e * s_estride + b0 * s_ld, s_ld, 1, nullptr, s_tile);
+  const int nb = B / COLS, nch = (A + kTRows - 1) / kTRows;
+  const int64_t e = blockIdx.x / (nb * nch);
+  const int b0 = (blockIdx.x / nch % nb) * COLS, a0 = blockIdx.x % nch * kTRows, n = min(kTRows, A - a0);
+  slab_t_quant<true, false, COLS, false, true>(x + (e * A + a0) * (int64_t)B + b0, B, n, n, q + e * q_estride + b0 * q_ld + a0, q_ld,
+                            s + e * s_estride + b0 * s_ld + a0 / kMxBlock, s_ld, 1, nullptr, s_tile);
 }
 
 // Both MX layouts of x [E][A][B] from one read: the row-wise one (q_r [E][A][B],
 // s_r [E][A][B / 32], as mx_quant_rows on [E A, B]) and the transposed one of
-// mx_quant_cols_t. Block per (e, COLS columns).
+// mx_quant_cols_t. Block per (e, COLS columns, 128 rows).
 template <int COLS>
 __global__ __launch_bounds__(4 * COLS) void mx_dual_cols_kernel(const uint16_t* __restrict__ x, int A, int B,
                                                            uint8_t* __restrict__ q, int64_t q_estride, int64_t q_ld,
                                                            uint8_t* __restrict__ s, int64_t s_estride, int64_t s_ld,
                                                            uint8_t* __restrict__ qr, uint8_t* __restrict__ sr) {
   __shared__ __attribute__((aligned(16))) uint32_t s_tile[kTRows * (COLS / 2)];
-  const int nb = B / COLS;
-  const int64_t e = blockIdx.x / nb;
-  const int b0 = (blockIdx.x % nb) * COLS;
-  const int64_t row0 = e * A;  // first row of expert e in the [E A, B] view
-  slab_t_quant<true, true, COLS>(x + row0 * B + b0, B, A, A, q + e * q_estride + b0 * q_ld, q_ld,
-                           s + e * s_estride + b0 * s_ld, s_ld, 1, nullptr, s_tile, qr + row0 * B + b0, B,
+  const int nb = B / COLS, nch = (A + kTRows - 1) / kTRows;
+  const int64_t e = blockIdx.x / (nb * nch);
+  const int b0 = (blockIdx.x / nch % nb) * COLS, a0 = blockIdx.x % nch * kTRows, n = min(kTRows, A - a0);
+  const int64_t row0 = e * A + a0;  // the chunk's first row in the [E A, B] view
+  slab_t_quant<true, true, COLS, false, true>(x + row0 * B + b0, B, n, n, q + e * q_estride + b0 * q_ld + a0, q_ld,
+                           s + e * s_estride + b0 * s_ld + a0 / kMxBlock, s_ld, 1, nullptr, s_tile, qr + row0 * B + b0, B,
                            sr + row0 * (B / kMxBlock) + b0 / kMxBlock, B / kMxBlock);
 }
 
 // x [R][C] with expert token groups (counts) -> q [C][Rpad] (group e at the
 // 128-aligned offset pstart_e, zero padded to ceil128(count_e)) and the scales
-// k-block major, s [Rpad / 32][C]. Block per (e, COLS columns); empty groups exit.
+// k-block major, s [Rpad / 32][C]. Block per (chunk of a group's rows, COLS columns).
 // With ROWS, the same read also writes the row-wise layout of the group's rows
 // (qr [R][C], sr [R][C / 32]).
 template <bool ROWS, int COLS, bool GATHER = false>
@@ -818,55 +902,44 @@ __global__ __launch_bounds__(4 * COLS) void mx_quant_tokens_t_kernel(const uint1
                                                                 uint8_t* __restrict__ sr, RowGather gather) {
   __shared__ __attribute__((aligned(16))) uint32_t s_tile[kTRows * (COLS / 2)];
   __shared__ int s_tmp[8];
-  __shared__ int s_seg[3];
-  // slab-major: the blocks running together share column slabs (1-4 % faster
-  // than expert-major at the Kimi shapes)
-  const int e = blockIdx.x % E;
-  const int c0 = (blockIdx.x / E) * COLS;
-  {
-    int cnt[4], pc[4], st[4], pst[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ee = threadIdx.x * 4 + i;
-      const int64_t c = ee < E ? counts[ee] : 0;
-      cnt[i] = c < 0 ? 0 : (int)(c > R ? R : c);
-      pc[i] = (cnt[i] + kMxPad - 1) / kMxPad * kMxPad;
-    }
-    block_exclusive_scan4(cnt, st, s_tmp);
-    block_exclusive_scan4(pc, pst, s_tmp);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (threadIdx.x * 4 + i == e) { s_seg[0] = st[i]; s_seg[1] = pst[i]; s_seg[2] = cnt[i]; }
-    __syncthreads();
-  }
-  const int seg0 = s_seg[0], pstart = s_seg[1];
-  int n = s_seg[2];
+  __shared__ GroupChunk s_gc;
+  const int n_chunks = (int)(R / kTRows) + E + kTailBlocks;
+  const int c0 = (blockIdx.x / n_chunks) * COLS;  // slab-major: blocks running together share column slabs
+  const GroupChunk gc = find_chunk(counts, R, E, blockIdx.x % n_chunks, s_tmp, &s_gc);
+  const int e = gc.e, seg0 = gc.seg0, pstart = gc.pstart, off = gc.off;
+  int n = gc.n;
   if ((int64_t)seg0 + n > R) n = (int)(R - seg0 > 0 ? R - seg0 : 0);
   const int n_out = (n + kMxPad - 1) / kMxPad * kMxPad;
-  if (e == E - 1 && (int64_t)pstart + n_out <= Rpad) {
-    // The columns past the last group, up to Rpad, belong to no group: zero them
-    // (and their scale rows) so that every byte of q and s is defined. Both ends
-    // are multiples of 32, so the rows' tails take 16-byte stores.
-    const int64_t end = (int64_t)pstart + n_out;
-    const int64_t tail16 = (Rpad - end) / 16;
-    for (int64_t i = threadIdx.x; i < COLS * tail16; i += 4 * COLS) {
+  if (e < 0) {
+    // The columns past the last group, up to Rpad, belong to no group: zero them (and
+    // their scale rows) so that every byte of q and s is defined. Both ends are multiples
+    // of 32, so the rows' tails take 16-byte stores. Up to E x 127 bytes of each row, by
+    // kTailBlocks blocks per slab: one block that also transposed the last group was the
+    // launch's last by a sixth of its time (64 groups, 32768 x 2304: 112 -> 93 us).
+    if (off >= kTailBlocks || (int64_t)pstart + n_out > Rpad) return;
+    constexpr int TC = COLS / kTailBlocks;
+    const int64_t end = (int64_t)pstart + n_out, tail16 = (Rpad - end) / 16;
+    const int64_t cb = c0 + off * TC;
+    for (int64_t i = threadIdx.x; i < TC * tail16; i += 4 * COLS) {
       const int64_t c = i / tail16, j = i - c * tail16;
-      *(uint4*)(q + (c0 + c) * Rpad + end + 16 * j) = make_uint4(0u, 0u, 0u, 0u);
+      *(uint4*)(q + (cb + c) * Rpad + end + 16 * j) = make_uint4(0u, 0u, 0u, 0u);
     }
-    if (threadIdx.x < COLS)
-      for (int64_t br = end / kMxBlock; br < Rpad / kMxBlock; ++br) s[br * C + c0 + threadIdx.x] = 0;
+    for (int64_t i = threadIdx.x; i < TC * (Rpad - end) / kMxBlock; i += 4 * COLS)
+      s[(end / kMxBlock + i / TC) * C + cb + i % TC] = 0;
+    return;
   }
-  if (n == 0 || (int64_t)pstart + n_out > Rpad) return;
+  if (n <= off || (int64_t)pstart + n_out > Rpad) return;
+  const int64_t r0 = (int64_t)seg0 + off;  // the chunk's first row, and its first token of q
+  const int64_t p0 = (int64_t)pstart + off;
   if constexpr (GATHER) {  // this slab's rows and columns of the gathered source
     gather.src += c0;
-    gather.idx += seg0;
-    if (gather.scale) gather.scale += seg0;
+    gather.idx += r0;
+    if (gather.scale) gather.scale += r0;
   }
-  slab_t_quant<true, ROWS, COLS, GATHER>(GATHER ? nullptr : x + (int64_t)seg0 * C + c0, C, n, n_out,
-                                 q + (int64_t)c0 * Rpad + pstart, Rpad, s + (int64_t)(pstart / kMxBlock) * C + c0, 1, C,
-                                 nullptr, s_tile, ROWS ? qr + (int64_t)seg0 * C + c0 : nullptr, C,
-                                 ROWS ? sr + (int64_t)seg0 * (C / kMxBlock) + c0 / kMxBlock : nullptr, C / kMxBlock,
-                                 gather, pstart % 128);
+  slab_t_quant<true, ROWS, COLS, GATHER, true>(GATHER ? nullptr : x + r0 * C + c0, C, min(n - off, kTRows), kTRows,
+                                 q + (int64_t)c0 * Rpad + p0, Rpad,
+                                 s + (p0 / kMxBlock) * C + c0, 1, C, nullptr, s_tile, ROWS ? qr + r0 * C + c0 : nullptr,
+                                 C, ROWS ? sr + r0 * (C / kMxBlock) + c0 / kMxBlock : nullptr, C / kMxBlock, gather);
 }
 
 // ---------------------------------------------------------------------------
@@ -1586,11 +1659,15 @@ static int quant_cols_t(const uint16_t* x, const float* col_amax, int32_t n_expe
       scale_expert_stride < b)
     return kErrInvalidArgument;
   if (!x || !q || !scale) return kErrInvalidArgument;
+  const bool one = col_amax != nullptr;
+  const int n_chunks = one ? (a + kTRows - 1) / kTRows : 1;
+  const auto k128 = one ? quant_cols_t_kernel<128, true> : quant_cols_t_kernel<128, false>;
+  const auto k64 = one ? quant_cols_t_kernel<64, true> : quant_cols_t_kernel<64, false>;
   if (b % 128 == 0)
-    hipLaunchKernelGGL(quant_cols_t_kernel<128>, dim3(n_experts * (b / 128)), dim3(512), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(k128, dim3(n_experts * (b / 128) * n_chunks), dim3(512), 0, stream, x, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, col_amax);
   else
-    hipLaunchKernelGGL(quant_cols_t_kernel<64>, dim3(n_experts * (b / 64)), dim3(256), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(k64, dim3(n_experts * (b / 64) * n_chunks), dim3(256), 0, stream, x, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, col_amax);
   return launch_status();
 }
@@ -1645,13 +1722,18 @@ static int quant_tokens_t(const uint16_t* x, const float* group_amax, const int6
   const bool g = gather.idx != nullptr;
   using kernel_t = void (*)(const uint16_t*, const int64_t*, int64_t, int, int, int64_t, uint8_t*, float*,
                             const float*, RowGather);
-  const kernel_t k128 = g ? quant_tokens_t_kernel<128, true> : quant_tokens_t_kernel<128, false>;
-  const kernel_t k64 = g ? quant_tokens_t_kernel<64, true> : quant_tokens_t_kernel<64, false>;
+  const bool one = group_amax != nullptr;
+  if (g && !one) return kErrInvalidArgument;
+  const kernel_t k128 = g ? quant_tokens_t_kernel<128, true, true>
+                          : (one ? quant_tokens_t_kernel<128, true> : quant_tokens_t_kernel<128, false>);
+  const kernel_t k64 = g ? quant_tokens_t_kernel<64, true, true>
+                         : (one ? quant_tokens_t_kernel<64, true> : quant_tokens_t_kernel<64, false>);
+  const int64_t n_blocks = one ? n_rows / kTRows + n_experts : n_experts;
   if (cols % 128 == 0)
-    hipLaunchKernelGGL(k128, dim3(n_experts * (cols / 128)), dim3(512), 0, stream, x, counts, n_rows, n_experts, cols,
+    hipLaunchKernelGGL(k128, dim3((unsigned)(n_blocks * (cols / 128))), dim3(512), 0, stream, x, counts, n_rows, n_experts, cols,
                        padded_rows, q, scale, group_amax, gather);
   else
-    hipLaunchKernelGGL(k64, dim3(n_experts * (cols / 64)), dim3(256), 0, stream, x, counts, n_rows, n_experts, cols,
+    hipLaunchKernelGGL(k64, dim3((unsigned)(n_blocks * (cols / 64))), dim3(256), 0, stream, x, counts, n_rows, n_experts, cols,
                        padded_rows, q, scale, group_amax, gather);
   return launch_status();
 }
@@ -1877,14 +1959,19 @@ MOE_API int moe_mxfp8_quant_cols_t(const uint16_t* x, int32_t n_experts, int32_t
   if (scale_row_stride < a / kMxBlock || scale_expert_stride < (int64_t)(b - 1) * scale_row_stride + a / kMxBlock)
     return kErrInvalidArgument;
   if (!x || !q || !scale) return kErrInvalidArgument;
+  const int n_chunks = (a + kTRows - 1) / kTRows;
   if (b % 128 == 0)
-    hipLaunchKernelGGL(mx_quant_cols_t_kernel<128>, dim3(n_experts * (b / 128)), dim3(512), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(mx_quant_cols_t_kernel<128>, dim3(n_experts * (b / 128) * n_chunks), dim3(512), 0, stream, x, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, scale_row_stride);
   else
-    hipLaunchKernelGGL(mx_quant_cols_t_kernel<64>, dim3(n_experts * (b / 64)), dim3(256), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(mx_quant_cols_t_kernel<64>, dim3(n_experts * (b / 64) * n_chunks), dim3(256), 0, stream, x, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, scale_row_stride);
   return launch_status();
 }
+
+// blocks per column slab: the 128-row chunks of a ragged routing, at most, and those of the
+// columns past the last group
+static int64_t token_blocks(int64_t n_rows, int n_experts) { return n_rows / kTRows + n_experts + kTailBlocks; }
 
 MOE_API int moe_mxfp8_quant_tokens_t(const uint16_t* x, const int64_t* counts, int64_t n_rows, int32_t n_experts,
                                      int32_t cols, int64_t padded_rows, uint8_t* q, uint8_t* scale,
@@ -1892,12 +1979,13 @@ MOE_API int moe_mxfp8_quant_tokens_t(const uint16_t* x, const int64_t* counts, i
   if (n_rows < 0 || n_experts < 1 || n_experts > kMaxE || cols < 64 || cols % 64) return kErrInvalidArgument;
   if (padded_rows < moe_mxfp8_padded_rows(n_rows, n_experts) || padded_rows % kMxPad) return kErrWorkspace;
   if (!x || !counts || !q || !scale) return kErrInvalidArgument;
+  const int64_t n_blocks = token_blocks(n_rows, n_experts);
   if (cols % 128 == 0)
-    hipLaunchKernelGGL((mx_quant_tokens_t_kernel<false, 128>), dim3(n_experts * (cols / 128)), dim3(512), 0, stream, x,
+    hipLaunchKernelGGL((mx_quant_tokens_t_kernel<false, 128>), dim3((unsigned)(n_blocks * (cols / 128))), dim3(512), 0, stream, x,
                        counts, n_rows, n_experts, cols, padded_rows, q, scale, (uint8_t*)nullptr, (uint8_t*)nullptr,
                        RowGather{});
   else
-    hipLaunchKernelGGL((mx_quant_tokens_t_kernel<false, 64>), dim3(n_experts * (cols / 64)), dim3(256), 0, stream, x,
+    hipLaunchKernelGGL((mx_quant_tokens_t_kernel<false, 64>), dim3((unsigned)(n_blocks * (cols / 64))), dim3(256), 0, stream, x,
                        counts, n_rows, n_experts, cols, padded_rows, q, scale, (uint8_t*)nullptr, (uint8_t*)nullptr,
                        RowGather{});
   return launch_status();
@@ -1913,11 +2001,12 @@ MOE_API int moe_mxfp8_quant_dual_cols(const uint16_t* x, int32_t n_experts, int3
   if (scale_row_stride < a / kMxBlock || scale_expert_stride < (int64_t)(b - 1) * scale_row_stride + a / kMxBlock)
     return kErrInvalidArgument;
   if (!x || !q || !scale || !q_rows || !scale_rows) return kErrInvalidArgument;
+  const int n_chunks = (a + kTRows - 1) / kTRows;
   if (b % 128 == 0)
-    hipLaunchKernelGGL(mx_dual_cols_kernel<128>, dim3(n_experts * (b / 128)), dim3(512), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(mx_dual_cols_kernel<128>, dim3(n_experts * (b / 128) * n_chunks), dim3(512), 0, stream, x, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, scale_row_stride, q_rows, scale_rows);
   else
-    hipLaunchKernelGGL(mx_dual_cols_kernel<64>, dim3(n_experts * (b / 64)), dim3(256), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(mx_dual_cols_kernel<64>, dim3(n_experts * (b / 64) * n_chunks), dim3(256), 0, stream, x, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, scale_row_stride, q_rows, scale_rows);
   return launch_status();
 }
@@ -1931,13 +2020,14 @@ static int mx_dual_tokens(const uint16_t* x, RowGather gather, const int64_t* co
   const bool g = gather.idx != nullptr;
   using kernel_t = void (*)(const uint16_t*, const int64_t*, int64_t, int, int, int64_t, uint8_t*, uint8_t*, uint8_t*,
                             uint8_t*, RowGather);
+  const int64_t n_blocks = token_blocks(n_rows, n_experts);
   const kernel_t k128 = g ? mx_quant_tokens_t_kernel<true, 128, true> : mx_quant_tokens_t_kernel<true, 128, false>;
   const kernel_t k64 = g ? mx_quant_tokens_t_kernel<true, 64, true> : mx_quant_tokens_t_kernel<true, 64, false>;
   if (cols % 128 == 0)
-    hipLaunchKernelGGL(k128, dim3(n_experts * (cols / 128)), dim3(512), 0, stream, x, counts, n_rows, n_experts, cols,
+    hipLaunchKernelGGL(k128, dim3((unsigned)(n_blocks * (cols / 128))), dim3(512), 0, stream, x, counts, n_rows, n_experts, cols,
                        padded_rows, q, scale, q_rows, scale_rows, gather);
   else
-    hipLaunchKernelGGL(k64, dim3(n_experts * (cols / 64)), dim3(256), 0, stream, x, counts, n_rows, n_experts, cols,
+    hipLaunchKernelGGL(k64, dim3((unsigned)(n_blocks * (cols / 64))), dim3(256), 0, stream, x, counts, n_rows, n_experts, cols,
                        padded_rows, q, scale, q_rows, scale_rows, gather);
   return launch_status();
 }
