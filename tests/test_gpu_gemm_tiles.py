@@ -91,3 +91,61 @@ def test_tiles(dev, name, oss):
         _close(a, b, f"gradient {i}", TOL[oss])
         if i and a.dim() == 3:
             assert not a[e // 2].any(), "gradient of an empty expert's weights"
+
+
+def _every_bf16(rows, cols):
+    """bf16 bit patterns over [rows, cols]: those in the reciprocal form's range first."""
+    bits = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    f = bits.float()
+    fast = (f >= -40.0) & (f <= 3.38e38)
+    v = torch.cat([bits[fast], bits[~fast]])
+    return v.repeat((rows * cols + v.numel() - 1) // v.numel())[:rows * cols].view(rows, cols)
+
+
+def test_gptoss_epilogues_every_bf16(dev):
+    """The gpt-oss epilogues on every bf16 value of g (infinities and NaNs included)
+    against torch's bf16 ops and their autograd: h from the g and u that gate_up returns,
+    and du from a one-hot dy, whose dh is mlp2's entries exactly, bit for bit; dg up to the
+    order of the three factors of torch's sigmoid backward, which can move the bf16 rounding
+    of that term, its product with alpha and the sum by one place (up to 2^-7) each."""
+    from torchtitan_amd import _lib
+
+    banner("gpt-oss epilogues, every bf16 g")
+    rows, d, h, limit, alpha = 256, 256, 256, 7.0, 1.702
+    gen = torch.Generator().manual_seed(13)
+    gt = _every_bf16(rows, h).to(dev)
+    u = (torch.randn(rows, h, generator=gen) * 4).bfloat16().to(dev)
+    counts = torch.tensor([rows], dtype=torch.int64, device=dev)
+    eye = torch.eye(rows, d, dtype=torch.bfloat16, device=dev)
+    st = torch.cuda.current_stream().cuda_stream
+
+    def act(g, v):
+        xg, xl = g.clamp(max=limit), v.clamp(min=-limit, max=limit)
+        return xg * torch.sigmoid(alpha * xg) * (xl + 1)
+
+    def same(a, b):
+        ok = (a.view(torch.int16) == b.view(torch.int16)) | (torch.isnan(a) & torch.isnan(b))
+        assert bool(ok.all()), int((~ok).sum())
+
+    w2 = (torch.randn(1, d, h, generator=gen) * 2).bfloat16().to(dev)
+    dgu = torch.empty(rows, 2 * h, dtype=torch.bfloat16, device=dev)
+    _lib.call("moe_grouped_gemm_oss_bwd_dgu", eye.data_ptr(), w2.data_ptr(), gt.data_ptr(), u.data_ptr(),
+              counts.data_ptr(), rows, 1, d, h, limit, dgu.data_ptr(), st)
+    gr, ur = gt.clone().requires_grad_(True), u.clone().requires_grad_(True)
+    act(gr, ur).backward(w2[0])
+    same(dgu[:, h:], ur.grad)
+    dg, want, gf = dgu[:, :h].float(), gr.grad.float(), gt.float()
+    assert torch.equal(torch.isfinite(dg), torch.isfinite(want))
+    xg, xl = gf.clamp(max=limit), u.float().clamp(min=-limit, max=limit)
+    sig = torch.sigmoid(alpha * xg)
+    term = (alpha * w2[0].float() * (xl + 1) * xg * sig * (1 - sig)).abs()
+    ok = (dg - want).abs() <= 2.0 ** -7 * (2 * torch.nan_to_num(term) + want.abs()) + 1e-30
+    assert bool((ok | ~torch.isfinite(want)).all()), int((~ok & torch.isfinite(want)).sum())
+
+    fin = torch.where(torch.isfinite(gt.float()), gt, torch.zeros_like(gt))
+    w1 = torch.stack([fin.t(), u.t()], dim=1).reshape(1, 2 * h, d).contiguous()  # glu 2 j, linear 2 j + 1
+    b1 = torch.randn(1, 2 * h, generator=gen).bfloat16().to(dev)
+    g2, u2, h2 = (torch.empty(rows, h, dtype=torch.bfloat16, device=dev) for _ in range(3))
+    _lib.call("moe_grouped_gemm_oss_gate_up", eye.data_ptr(), w1.data_ptr(), b1.data_ptr(), counts.data_ptr(), rows, 1,
+              d, h, limit, g2.data_ptr(), u2.data_ptr(), h2.data_ptr(), st)
+    same(h2, act(g2, u2))

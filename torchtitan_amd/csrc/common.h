@@ -57,6 +57,14 @@ __device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
 }
 
+// The same roundings for values that are not stored: a NaN stays a NaN, whichever
+// (v_cvt_pk_bf16_f32 keeps every one of the fp32 NaNs, checked on the GPU), and becomes the
+// canonical one where the value computed from it is stored. Two instructions less per value.
+__device__ __forceinline__ uint32_t pack_bf2_mid(float lo, float hi) {
+  const f32x2_t v = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+}
+
 // silu(g) = g / d and sigmoid(g) = 1 / d with d = 1 + exp(-g), the quotients rounded
 // as IEEE division rounds them (torch's kernels divide), without the general
 // division's scaling and fix-up steps: the hardware reciprocal estimate refined by one
@@ -122,6 +130,9 @@ __device__ __forceinline__ uint4 span64_lds(uint2 lo, uint2 hi, int lane) {
 }
 __device__ __forceinline__ uint2 pack4(const float (&v)[4]) {
   return make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+}
+__device__ __forceinline__ uint2 pack4_mid(const float (&v)[4]) {
+  return make_uint2(pack_bf2_mid(v[0], v[1]), pack_bf2_mid(v[2], v[3]));
 }
 
 

@@ -105,21 +105,41 @@ struct GemmParams {
   float alpha;         // 1.702
 };
 
-__device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
-__device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
-
 // Expert epilogue variants: the SwiGLU of moe.py:53-70 and gpt-oss's biased,
 // clamped SwiGLU with interleaved mlp1 rows (gpt_oss/moe.py:43-52, 92-122).
 enum ExpertAct : int { kSwiGLU = 0, kOssGLU = 1 };
 
-// gpt-oss activation on bf16 values g (glu), u (linear), every op rounded to
-// bf16 as the reference's bf16 tensor ops: clamp(g, max=L), clamp(u, -L, L),
-// g * sigmoid(alpha g), times (u + 1). Returns the last product unrounded.
-__device__ __forceinline__ float oss_glu(float g, float u, float L, float alpha) {
-  const float xg = g > L ? L : g;                      // NaN passes, as torch.clamp
-  const float xl = u < -L ? -L : (u > L ? L : u);
-  const float s = round_bf(sigmoid_f(round_bf(xg * alpha)));
-  return round_bf(xg * s) * round_bf(xl + 1.0f);
+// gpt-oss activation on pairs of bf16 values g (glu), u (linear), every op rounded to
+// bf16 as the reference's bf16 tensor ops: xg = clamp(g, max=L), xl = clamp(u, -L, L),
+// s = sigmoid(alpha xg), og = xg s, lin = xl + 1. The pair's two roundings are one
+// conversion, and the sigmoid divides in the reciprocal form where both lie in its range
+// (silu_sig: equal to IEEE division for every bf16 argument). The epilogues are VALU-bound;
+// with one canonicalizing conversion per value and a division gate_up took 670 us and dgu
+// 510 us at 32 experts, 16384 rows, 2880 / 2880, now 642 and 478.
+struct OssGlu { float xg[2], s[2], og[2], lin[2]; };
+__device__ __forceinline__ void oss_pair(float (&r)[2], float a, float b) {
+  const uint32_t w = pack_bf2_mid(a, b);
+  r[0] = bf_lo(w);
+  r[1] = bf_hi(w);
+}
+__device__ __forceinline__ OssGlu oss_glu(float g0, float g1, float u0, float u1, float L, float alpha) {
+  OssGlu o;
+  const float g[2] = {g0, g1}, u[2] = {u0, u1};
+  float xl[2], z[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    o.xg[i] = g[i] > L ? L : g[i];                         // NaN passes, as torch.clamp
+    xl[i] = u[i] < -L ? -L : (u[i] > L ? L : u[i]);
+  }
+  oss_pair(z, o.xg[0] * alpha, o.xg[1] * alpha);
+  const float d0 = silu_den(z[0]), d1 = silu_den(z[1]);
+  if (silu_fast_wave(fminf(z[0], z[1]), fmaxf(z[0], z[1])))
+    oss_pair(o.s, silu_sig<true>(z[0], d0).sig, silu_sig<true>(z[1], d1).sig);
+  else
+    oss_pair(o.s, silu_sig<false>(z[0], d0).sig, silu_sig<false>(z[1], d1).sig);
+  oss_pair(o.og, o.xg[0] * o.s[0], o.xg[1] * o.s[1]);
+  oss_pair(o.lin, xl[0] + 1.0f, xl[1] + 1.0f);
+  return o;
 }
 template <int MODE>
 struct ModeTraits {
@@ -467,8 +487,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void grouped_gemm_kernel(GemmParams p
         if constexpr (kParkRegs) {
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
-            park[i][j][0] = pack_bf2(acc[i][j][0], acc[i][j][1]);
-            park[i][j][1] = pack_bf2(acc[i][j][2], acc[i][j][3]);
+            park[i][j][0] = pack_bf2_mid(acc[i][j][0], acc[i][j][1]);
+            park[i][j][1] = pack_bf2_mid(acc[i][j][2], acc[i][j][3]);
           }
         } else {
           // 64-byte row pieces of the dx rows (read back the same way in the epilogue)
@@ -477,7 +497,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void grouped_gemm_kernel(GemmParams p
             const float lo[4] = {acc[i][2 * jp][0], acc[i][2 * jp][1], acc[i][2 * jp][2], acc[i][2 * jp][3]};
             const float hi[4] = {acc[i][2 * jp + 1][0], acc[i][2 * jp + 1][1], acc[i][2 * jp + 1][2],
                                  acc[i][2 * jp + 1][3]};
-            const uint4 sv = span64(pack4(lo), pack4(hi), lane);
+            const uint4 sv = span64(pack4_mid(lo), pack4_mid(hi), lane);
             const int n = nt * BN + wn * WN + jp * 32 + 8 * (lane >> 4);
             if (r < seg1 && (!TAIL || n < D)) *(uint4*)(p.out_dx + (int64_t)r * D + n) = sv;
           }
@@ -636,20 +656,23 @@ __global__ __launch_bounds__(NW * 64, OCC) void grouped_gemm_kernel(GemmParams p
 #pragma unroll
               for (int q2 = 0; q2 < 2; ++q2) {
                 const int q = 2 * q2;
-                uint32_t gw = pack_bf2(acc[i][2 * jj][q], acc[i][2 * jj][q + 1]);
-                uint32_t uw = pack_bf2(acc[i][2 * jj + 1][q], acc[i][2 * jj + 1][q + 1]);
+                uint32_t gw, uw;
                 if constexpr (ACT == kOssGLU) {
+                  gw = pack_bf2_mid(acc[i][2 * jj][q], acc[i][2 * jj][q + 1]);
+                  uw = pack_bf2_mid(acc[i][2 * jj + 1][q], acc[i][2 * jj + 1][q + 1]);
                   // h1 = bf16(x . mlp1^T) + bias (bf16 add), then the clamped SwiGLU;
                   // bias word of column c: (glu, linear)
                   const uint4 bw = bias1[jj];
                   const uint32_t bb[4] = {bw.x, bw.y, bw.z, bw.w};
                   gw = pack_bf2(bf_lo(gw) + bf_lo(bb[q]), bf_hi(gw) + bf_lo(bb[q + 1]));
                   uw = pack_bf2(bf_lo(uw) + bf_hi(bb[q]), bf_hi(uw) + bf_hi(bb[q + 1]));
-                  hq[q2] = pack_bf2(oss_glu(bf_lo(gw), bf_lo(uw), p.limit, p.alpha),
-                                    oss_glu(bf_hi(gw), bf_hi(uw), p.limit, p.alpha));
+                  const OssGlu o = oss_glu(bf_lo(gw), bf_hi(gw), bf_lo(uw), bf_hi(uw), p.limit, p.alpha);
+                  hq[q2] = pack_bf2(o.og[0] * o.lin[0], o.og[1] * o.lin[1]);
                 } else {
+                  gw = pack_bf2(acc[i][2 * jj][q], acc[i][2 * jj][q + 1]);
+                  uw = pack_bf2(acc[i][2 * jj + 1][q], acc[i][2 * jj + 1][q + 1]);
                   const float g0 = bf_lo(gw), g1 = bf_hi(gw);
-                  const uint32_t sw = pack_bf2(silu_sig<kFast>(g0, silu_den(g0)).silu,
+                  const uint32_t sw = pack_bf2_mid(silu_sig<kFast>(g0, silu_den(g0)).silu,
                                                silu_sig<kFast>(g1, silu_den(g1)).silu);  // bf16(silu(g))
                   hq[q2] = pack_bf2(bf_lo(sw) * bf_lo(uw), bf_hi(sw) * bf_hi(uw));
                 }
@@ -703,7 +726,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void grouped_gemm_kernel(GemmParams p
               const float lo[4] = {acc[i][2 * jp][0], acc[i][2 * jp][1], acc[i][2 * jp][2], acc[i][2 * jp][3]};
               const float hi[4] = {acc[i][2 * jp + 1][0], acc[i][2 * jp + 1][1], acc[i][2 * jp + 1][2],
                                    acc[i][2 * jp + 1][3]};
-              const uint4 sv = span64(pack4(lo), pack4(hi), lane);
+              const uint4 sv = span64(pack4_mid(lo), pack4_mid(hi), lane);
               const int n = nt * BN + wn * WN + jp * 32 + g8;
               if (TAIL && n >= D) continue;
               uint16_t* dst = outp + (int64_t)r * D + n;
@@ -725,17 +748,19 @@ __global__ __launch_bounds__(NW * 64, OCC) void grouped_gemm_kernel(GemmParams p
               float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
               if (MODE == kFwdDown && ACT == kOssGLU) {  // bf16(h . mlp2^T) + mlp2_bias (bf16 add)
                 const uint2 bw = bias2[j];
-                v[0] = round_bf(v[0]) + bf_lo(bw.x);
-                v[1] = round_bf(v[1]) + bf_hi(bw.x);
-                v[2] = round_bf(v[2]) + bf_lo(bw.y);
-                v[3] = round_bf(v[3]) + bf_hi(bw.y);
+                const uint2 rv = pack4_mid(v);
+                v[0] = bf_lo(rv.x) + bf_lo(bw.x);
+                v[1] = bf_hi(rv.x) + bf_hi(bw.x);
+                v[2] = bf_lo(rv.y) + bf_lo(bw.y);
+                v[3] = bf_hi(rv.y) + bf_hi(bw.y);
               }
               if constexpr (MODE == kBwdDx && ACT == kSwiGLU && kParkRegs) {
                 const uint2 pw = make_uint2(park[i][j][0], park[i][j][1]);
-                v[0] = bf_lo(pw.x) + round_bf(v[0]);
-                v[1] = bf_hi(pw.x) + round_bf(v[1]);
-                v[2] = bf_lo(pw.y) + round_bf(v[2]);
-                v[3] = bf_hi(pw.y) + round_bf(v[3]);
+                const uint2 rv = pack4_mid(v);
+                v[0] = bf_lo(pw.x) + bf_lo(rv.x);
+                v[1] = bf_hi(pw.x) + bf_hi(rv.x);
+                v[2] = bf_lo(pw.y) + bf_lo(rv.y);
+                v[3] = bf_hi(pw.y) + bf_hi(rv.y);
               }
               pv[h2] = pack4(v);
             }
@@ -775,7 +800,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void grouped_gemm_kernel(GemmParams p
             const float lo[4] = {acc[i][2 * jp][0], acc[i][2 * jp][1], acc[i][2 * jp][2], acc[i][2 * jp][3]};
             const float hi[4] = {acc[i][2 * jp + 1][0], acc[i][2 * jp + 1][1], acc[i][2 * jp + 1][2],
                                  acc[i][2 * jp + 1][3]};
-            const uint4 sdh = span64(pack4(lo), pack4(hi), lane);
+            const uint4 sdh = span64(pack4_mid(lo), pack4_mid(hi), lane);
             const int hh = nt * BN + wn * WN + jp * 32 + g8;
             if (TAIL && hh >= H) continue;
             const uint4 gw = gbuf[0][jp];
@@ -803,8 +828,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void grouped_gemm_kernel(GemmParams p
                   f0 = silu_sig<false>(gv, d0);
                   f1 = silu_sig<false>(gv1, d1);
                 }
-                const uint32_t slw = pack_bf2(f0.silu, f1.silu);   // bf16(silu(g))
-                const uint32_t dsw = pack_bf2(dh * uv, dh1 * uv1);  // bf16(dh . u)
+                const uint32_t slw = pack_bf2_mid(f0.silu, f1.silu);   // bf16(silu(g))
+                const uint32_t dsw = pack_bf2_mid(dh * uv, dh1 * uv1);  // bf16(dh . u)
                 du[q] = dh * bf_lo(slw);
                 du[q + 1] = dh1 * bf_hi(slw);
                 const float sg = f0.sig, sg1 = f1.sig;
@@ -812,18 +837,23 @@ __global__ __launch_bounds__(NW * 64, OCC) void grouped_gemm_kernel(GemmParams p
                 dg[q + 1] = bf_hi(dsw) * sg1 * (1.0f + gv1 * (1.0f - sg1));
               } else {
                 // autograd of oss_glu, each bf16 op's gradient rounded to bf16
+                if (q & 1) continue;
                 const float L = p.limit, al = p.alpha;
-                const float xg = gv > L ? L : gv;
-                const float xl = uv < -L ? -L : (uv > L ? L : uv);
-                const float s = round_bf(sigmoid_f(round_bf(xg * al)));
-                const float og = round_bf(xg * s);
-                const float da = round_bf(dh * round_bf(xl + 1.0f));  // d(glu output)
-                const float dl = round_bf(dh * og);                    // d(linear + 1)
-                const float ds = round_bf(da * xg);                    // d(sigmoid output)
-                const float dz = round_bf((ds * (1.0f - s)) * s);      // sigmoid_backward
-                const float dxg = round_bf(da * s) + round_bf(dz * al);
-                dg[q] = gv <= L ? dxg : 0.f;                           // clamp(max=L) backward
-                du[q] = (uv >= -L && uv <= L) ? dl : 0.f;              // clamp(-L, L) backward
+                const float dhp[2] = {dh, bf_hi(dhw[q >> 1])}, gp[2] = {gv, bf_hi(gww[q >> 1])},
+                            up[2] = {uv, bf_hi(uww[q >> 1])};
+                const OssGlu o = oss_glu(gp[0], gp[1], up[0], up[1], L, al);
+                float da[2], dl[2], ds[2], dz[2], a1[2], a2[2];
+                oss_pair(da, dhp[0] * o.lin[0], dhp[1] * o.lin[1]);  // d(glu output)
+                oss_pair(dl, dhp[0] * o.og[0], dhp[1] * o.og[1]);    // d(linear + 1)
+                oss_pair(ds, da[0] * o.xg[0], da[1] * o.xg[1]);      // d(sigmoid output)
+                oss_pair(dz, (ds[0] * (1.0f - o.s[0])) * o.s[0], (ds[1] * (1.0f - o.s[1])) * o.s[1]);  // sigmoid_backward
+                oss_pair(a1, da[0] * o.s[0], da[1] * o.s[1]);
+                oss_pair(a2, dz[0] * al, dz[1] * al);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                  dg[q + i] = gp[i] <= L ? a1[i] + a2[i] : 0.f;                 // clamp(max=L) backward
+                  du[q + i] = (up[i] >= -L && up[i] <= L) ? dl[i] : 0.f;        // clamp(-L, L) backward
+                }
               }
             }
             const int64_t o2 = (int64_t)r * (2 * H) + hh;
@@ -930,7 +960,8 @@ static void launch_cfg(const GemmParams& p, int64_t R, hipStream_t stream) {
 //                  has more than one tile of rows (the narrow tile streams weights faster)
 //                  128 x 512                                   1.73, where D is a multiple of
 //                  512 (its w1 half is parked in the dx rows: a partial tile wastes that
-//                  traffic too); the gpt-oss dx parks nothing and takes it at any D
+//                  traffic too); the gpt-oss dx parks nothing and takes it at any D, and
+//                  has the 256 x 256 tile, 1.62 (7 % slower where w1's half is parked)
 //                  128 x 256 of four waves, 2 per CU           1.95 (512 slots)
 //  dW              256 x 256, 32-wide, 3 stages; 128 x 128 of four waves, 2 per CU,
 //                  only where the wide tiles leave half the chip idle (the smaller tile
@@ -980,7 +1011,14 @@ static void launch_mode(const GemmParams& p, int64_t R, hipStream_t stream) {
                  c384 = (several ? 1.45 : 1.55) * rounds(m128 * n_tiles(p.D, 384), 1),
                  c512 = ACT == kOssGLU || p.D % 512 == 0 ? 1.73 * rounds(m128 * n_tiles(p.D, 512), 1) : INFINITY,
                  c_two = 1.95 * rounds(m128 * n_tiles(p.D, 256), 2);
-    const double best = fmin(fmin(c256, c384), fmin(c512, c_two));
+    const double c_tall = ACT == kOssGLU ? 1.62 * rounds(m256 * n_tiles(p.D, 256), 1) : INFINITY;
+    const double best = fmin(fmin(c256, c384), fmin(fmin(c512, c_tall), c_two));
+    if constexpr (ACT == kOssGLU) {
+      if (best == c_tall) {
+        launch_cfg<MODE, 8, 4, 4, 8, 3, false, 1, ACT>(p, R, stream);
+        return;
+      }
+    }
     if (best == c384) launch_cfg<MODE, 8, 2, 4, 6, 3, false, 1, ACT>(p, R, stream);
     else if (best == c512) launch_cfg<MODE, 8, 2, 4, 8, 3, false, 1, ACT>(p, R, stream);
     else if (best == c256) launch_cfg<MODE, 8, 2, 4, 4, 3, false, 1, ACT>(p, R, stream);
