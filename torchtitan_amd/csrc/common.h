@@ -148,6 +148,10 @@ template <> struct Chunk<uint16_t> {
   static __device__ __forceinline__ uint4 pack(const float (&f)[8]) {
     return make_uint4(pack_bf2(f[0], f[1]), pack_bf2(f[2], f[3]), pack_bf2(f[4], f[5]), pack_bf2(f[6], f[7]));
   }
+  static __device__ __forceinline__ uint4 pack_mid(const float (&f)[8]) {
+    return make_uint4(pack_bf2_mid(f[0], f[1]), pack_bf2_mid(f[2], f[3]), pack_bf2_mid(f[4], f[5]),
+                      pack_bf2_mid(f[6], f[7]));
+  }
   static __device__ __forceinline__ float round(float f) { return round_bf(f); }
 };
 template <> struct Chunk<float> {
@@ -159,6 +163,7 @@ template <> struct Chunk<float> {
   static __device__ __forceinline__ uint4 pack(const float (&f)[4]) {
     return make_uint4(__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3]));
   }
+  static __device__ __forceinline__ uint4 pack_mid(const float (&f)[4]) { return pack(f); }
   static __device__ __forceinline__ float round(float f) { return f; }
 };
 

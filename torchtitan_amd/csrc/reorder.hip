@@ -242,6 +242,11 @@ __global__ __launch_bounds__(256) void scatter_kernel(ScatterParams p) {
 // ---------------------------------------------------------------------------
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
+__device__ __forceinline__ uint4 nt_load(const void* p) {
+  const u32x4_t w = __builtin_nontemporal_load((const u32x4_t*)p);
+  return make_uint4(w.x, w.y, w.z, w.w);
+}
+
 template <typename T>
 __device__ __forceinline__ uint4 scale_chunk(uint4 v, float s) {
   constexpr int n = Chunk<T>::kN;
@@ -250,6 +255,18 @@ __device__ __forceinline__ uint4 scale_chunk(uint4 v, float s) {
 #pragma unroll
   for (int i = 0; i < n; ++i) f[i] = f[i] * s;
   return Chunk<T>::pack(f);
+}
+
+// the same for a product that is not stored, rounded by itself also where it is added next
+template <typename T>
+__device__ __forceinline__ uint4 scale_chunk_mid(uint4 v, float s) {
+#pragma clang fp contract(off)
+  constexpr int n = Chunk<T>::kN;
+  float f[n];
+  Chunk<T>::unpack(v, f);
+#pragma unroll
+  for (int i = 0; i < n; ++i) f[i] = f[i] * s;
+  return Chunk<T>::pack_mid(f);
 }
 
 template <typename T>
@@ -298,6 +315,9 @@ __global__ __launch_bounds__(256) void expand_rows_kernel(const T* __restrict__ 
 // sorted index_put with accumulate); r_k = routed[pos_k], or
 // round(routed[pos_k] * score) when the score is applied after the experts
 // (moe.py:465-469). Without a shared expert the sum starts from zero.
+// Bound by reading the routed rows, once each: their loads do not keep them in the caches
+// (timed after the kernel that writes them: 154 -> 134 us for 604 MB of
+// bf16 rows, 132 -> 105 for 537 MB of fp32, 74 -> 64 for 302 MB, 18 for 75 MB either way).
 template <typename T, int MAXK>
 __global__ __launch_bounds__(256) void combine_kernel(const T* __restrict__ shared_out,
                                                       const T* __restrict__ routed,
@@ -326,7 +346,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const T* __restrict__ shar
     uint4 v[MAXK];
 #pragma unroll
     for (int k = 0; k < MAXK; ++k)
-      v[k] = k < K ? *(const uint4*)(routed + (int64_t)pos[k] * D + ch * n) : make_uint4(0, 0, 0, 0);
+      v[k] = k < K ? nt_load(routed + (int64_t)pos[k] * D + ch * n) : make_uint4(0, 0, 0, 0);
 #pragma unroll
     for (int k = 0; k < MAXK; ++k) {
       if (k < K) {
@@ -342,16 +362,28 @@ __global__ __launch_bounds__(256) void combine_kernel(const T* __restrict__ shar
   }
 }
 
+// The wavefront's index in its block for the kernels of a wavefront per token, as a scalar:
+// the token's positions, scores and row addresses are then scalar loads and registers
+// (permute_bwd 120 -> 74 vector registers, six waves a SIMD instead of four). Past 16 experts
+// a token they no longer fit the scalar registers (over 2000 spills) and stay per lane.
+template <int MAXK>
+__device__ __forceinline__ int token_wave() {
+  const int wv = threadIdx.x >> 6;
+  return MAXK <= 16 ? __builtin_amdgcn_readfirstlane(wv) : wv;
+}
+
 // Backward of the combine when the score is applied after the experts:
 //   grad_routed[pos] = round(grad_out[t] * s[pos]);  grad_s[pos] = sum_d grad_out[t,d] * routed[pos,d]
-// One wavefront per token.
+// One wavefront per token, its positions scalar for K in 9..16 (4096 tokens of 2304, K = 16:
+// 178 -> 141 us); with fewer they fit the vector registers and scalar ones win 7 % at 1024
+// columns but lose 3 to 5 % from 2304 on.
 template <typename T, int MAXK>
 __global__ __launch_bounds__(256) void combine_bwd_scored_kernel(
     const T* __restrict__ grad_out, const T* __restrict__ routed, const int32_t* __restrict__ tok_pos,
     const float* __restrict__ scores_sorted, int64_t n_tokens, int D, int K, T* __restrict__ grad_routed,
     float* __restrict__ grad_scores) {
   constexpr int n = Chunk<T>::kN;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = sizeof(T) == 2 && MAXK == 16 ? token_wave<MAXK>() : threadIdx.x >> 6;
   const int cpr = D / n;
   for (int64_t t = (int64_t)blockIdx.x * 4 + wv; t < n_tokens; t += (int64_t)gridDim.x * 4) {
     float part[MAXK];
@@ -390,14 +422,17 @@ __global__ __launch_bounds__(256) void combine_bwd_scored_kernel(
 //   rounding to the row type after every add when round_each (ATen's
 //   index_put with accumulate on row slices), else once at the end;
 //   grad_s[pos] = sum_d g * x[t]   (only when scores are given).
-// One wavefront per token.
-template <typename T, int MAXK>
+// One wavefront per token. Bound by reading the gradient rows; a kernel per rounding and
+// scoring instead of branches at every add, scalar positions and rows read past the caches
+// once they exceed them (STREAM): 16384 tokens of 2304 in bf16, K = 8, 171 -> 135 us
+// (755 MB, 5.6 TB/s); 4096 such tokens with K = 16 105 -> 73, with K = 20 215 -> 148.
+template <typename T, int MAXK, bool SCORED, bool ROUND, bool STREAM>
 __global__ __launch_bounds__(256) void permute_bwd_kernel(
     const T* __restrict__ grad_routed, const T* __restrict__ x, const int32_t* __restrict__ tok_pos,
-    const float* __restrict__ scores_sorted, int64_t n_tokens, int D, int K, int round_each,
-    T* __restrict__ grad_x, float* __restrict__ grad_scores) {
+    const float* __restrict__ scores_sorted, int64_t n_tokens, int D, int K, T* __restrict__ grad_x,
+    float* __restrict__ grad_scores) {
   constexpr int n = Chunk<T>::kN;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = token_wave<MAXK>();
   const int cpr = D / n;
   for (int64_t t = (int64_t)blockIdx.x * 4 + wv; t < n_tokens; t += (int64_t)gridDim.x * 4) {
     float part[MAXK];
@@ -407,14 +442,14 @@ __global__ __launch_bounds__(256) void permute_bwd_kernel(
     for (int k = 0; k < MAXK; ++k) {
       part[k] = 0.f;
       pos[k] = (k < K) ? tok_pos[t * K + k] : 0;
-      sc[k] = (k < K && scores_sorted) ? scores_sorted[pos[k]] : 1.0f;
+      if constexpr (SCORED) sc[k] = (k < K) ? scores_sorted[pos[k]] : 1.0f;
     }
     // row chunks loaded in batches of HK: all eight at once for K <= 8 (4 % faster
     // than two batches of four at the Kimi shape), two batches above
     constexpr int HK = MAXK <= 8 ? MAXK : MAXK / 2, NB = MAXK / HK;
     for (int ch = lane; ch < cpr; ch += kWave) {
       uint4 xv = make_uint4(0, 0, 0, 0);
-      if (scores_sorted) xv = *(const uint4*)(x + t * D + ch * n);
+      if constexpr (SCORED) xv = *(const uint4*)(x + t * D + ch * n);
       float a[n];
 #pragma unroll
       for (int i = 0; i < n; ++i) a[i] = 0.f;
@@ -424,27 +459,31 @@ __global__ __launch_bounds__(256) void permute_bwd_kernel(
 #pragma unroll
         for (int kk = 0; kk < HK; ++kk) {
           const int k = h * HK + kk;
-          gk[kk] = (k < K) ? *(const uint4*)(grad_routed + (int64_t)pos[k] * D + ch * n) : make_uint4(0, 0, 0, 0);
+          if (k >= K) continue;
+          const T* row = grad_routed + (int64_t)pos[k] * D + ch * n;
+          if constexpr (STREAM) gk[kk] = nt_load(row);
+          else gk[kk] = *(const uint4*)row;
         }
 #pragma unroll
         for (int kk = 0; kk < HK; ++kk) {
           const int k = h * HK + kk;
           if (k < K) {
             uint4 g = gk[kk];
-            if (scores_sorted) {
+            if constexpr (SCORED) {
               part[k] += dot_chunk<T>(g, xv);
-              g = scale_chunk<T>(g, sc[k]);
+              g = scale_chunk_mid<T>(g, sc[k]);
             }
             float f[n];
             Chunk<T>::unpack(g, f);
 #pragma unroll
-            for (int i = 0; i < n; ++i) a[i] = round_each ? Chunk<T>::round(a[i] + f[i]) : (a[i] + f[i]);
+            for (int i = 0; i < n; ++i) a[i] = a[i] + f[i];
+            if constexpr (ROUND) Chunk<T>::unpack(Chunk<T>::pack_mid(a), a);
           }
         }
       }
       *(uint4*)(grad_x + t * D + ch * n) = Chunk<T>::pack(a);
     }
-    if (scores_sorted && grad_scores) {
+    if constexpr (SCORED) {
 #pragma unroll
       for (int k = 0; k < MAXK; ++k) {
         if (k < K) {
@@ -463,6 +502,17 @@ __global__ __launch_bounds__(256) void gather_scores_kernel(const float* __restr
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
     out[i] = 0.0f + grad_sorted[slot_pos[i]];
+}
+
+// Sorted rows (all n_tokens * top_k of them) past this many bytes go through the 256 MB cache
+// in front of HBM without being kept there: they push each other out before the next kernel
+// reads them. Each kernel timed with the copy that writes its rows or reads them next, kept /
+// not kept: expand 18 / 23 us at 75 MB, 23 / 33 at 151, 57 / 48 at 201, 78 / 70 at 302,
+// 158 / 144 at 604; permute_bwd 35 / 33, 46 / 43, 80 / 67, 169 / 145 from 151 MB on.
+constexpr int64_t kStreamBytes = 176ll << 20;
+template <typename T>
+static bool streamed(int64_t n_tokens, int dim, int top_k) {
+  return n_tokens * top_k * dim * (int64_t)sizeof(T) > kStreamBytes;
 }
 
 static int stream_grid(int64_t work, int per_block = 256, int cap = 8192) {
@@ -571,15 +621,11 @@ static int check_row_args(int64_t n_tokens, int32_t dim, int32_t top_k, int32_t 
   return kErrInvalidArgument;
 }
 
-// stream: nontemporal stores, for the permute, whose rows the next kernel reads
-// from HBM anyway (measured 0.146 -> 0.123 ms at the Kimi shape); the combine
-// backward keeps ordinary stores (its output is read back at once: 0.118 -> 0.133
-// ms with streamed stores)
 template <typename T>
 static void launch_expand(const void* src, int64_t n_tokens, int dim, int top_k, const int32_t* slot_pos,
-                          const float* scores, void* out, bool stream_stores, hipStream_t stream) {
+                          const float* scores, void* out, hipStream_t stream) {
   const dim3 grid(stream_grid(n_tokens * (dim / Chunk<T>::kN)));
-  if (stream_stores)
+  if (streamed<T>(n_tokens, dim, top_k))
     hipLaunchKernelGGL((expand_rows_kernel<T, true>), grid, dim3(256), 0, stream, (const T*)src, n_tokens, dim,
                        top_k, slot_pos, scores, (T*)out);
   else
@@ -603,20 +649,30 @@ static void launch_combine(const void* shared_out, const void* routed, const int
                        (const T*)routed, tok_pos, scores, n_tokens, dim, top_k, (T*)out);
 }
 
+template <typename T, int MAXK, bool STREAM>
+static void launch_permute_bwd(const void* grad_routed, const void* x, const int32_t* tok_pos,
+                               const float* scores, int64_t n_tokens, int dim, int top_k, int round_each,
+                               void* grad_x, float* grad_scores, hipStream_t stream) {
+  constexpr bool kRounds = sizeof(T) == 2;  // fp32 rows have no rounding between the adds
+  const bool round = kRounds && round_each;
+  auto* kernel = scores ? (round ? permute_bwd_kernel<T, MAXK, true, kRounds, STREAM>
+                                 : permute_bwd_kernel<T, MAXK, true, false, STREAM>)
+                        : (round ? permute_bwd_kernel<T, MAXK, false, kRounds, STREAM>
+                                 : permute_bwd_kernel<T, MAXK, false, false, STREAM>);
+  hipLaunchKernelGGL(kernel, dim3(stream_grid(n_tokens, 4, 16384)), dim3(256), 0, stream, (const T*)grad_routed,
+                     (const T*)x, tok_pos, scores, n_tokens, dim, top_k, (T*)grad_x, grad_scores);
+}
+
 template <typename T>
 static void launch_permute_bwd(const void* grad_routed, const void* x, const int32_t* tok_pos,
                                const float* scores, int64_t n_tokens, int dim, int top_k, int round_each,
                                void* grad_x, float* grad_scores, hipStream_t stream) {
-  const dim3 grid(stream_grid(n_tokens, 4, 16384));
-  if (top_k <= 8)
-    hipLaunchKernelGGL((permute_bwd_kernel<T, 8>), grid, dim3(256), 0, stream, (const T*)grad_routed,
-                       (const T*)x, tok_pos, scores, n_tokens, dim, top_k, round_each, (T*)grad_x, grad_scores);
-  else if (top_k <= 16)
-    hipLaunchKernelGGL((permute_bwd_kernel<T, 16>), grid, dim3(256), 0, stream, (const T*)grad_routed,
-                       (const T*)x, tok_pos, scores, n_tokens, dim, top_k, round_each, (T*)grad_x, grad_scores);
-  else
-    hipLaunchKernelGGL((permute_bwd_kernel<T, kMaxTopK>), grid, dim3(256), 0, stream, (const T*)grad_routed,
-                       (const T*)x, tok_pos, scores, n_tokens, dim, top_k, round_each, (T*)grad_x, grad_scores);
+  // (unscored fp32 rows are read as fast either way: 130 / 132 us for 537 MB)
+  const bool nt = (scores || sizeof(T) == 2) && streamed<T>(n_tokens, dim, top_k);
+  auto* launch = top_k <= 8    ? (nt ? launch_permute_bwd<T, 8, true> : launch_permute_bwd<T, 8, false>)
+                 : top_k <= 16 ? (nt ? launch_permute_bwd<T, 16, true> : launch_permute_bwd<T, 16, false>)
+                               : (nt ? launch_permute_bwd<T, kMaxTopK, true> : launch_permute_bwd<T, kMaxTopK, false>);
+  launch(grad_routed, x, tok_pos, scores, n_tokens, dim, top_k, round_each, grad_x, grad_scores, stream);
 }
 
 template <typename T>
@@ -643,9 +699,9 @@ MOE_API int moe_permute(const void* x, const int32_t* slot_pos, const float* sco
   if (n_tokens == 0) return kOk;
   if (!x || !slot_pos || !routed_input) return kErrInvalidArgument;
   if (dtype == MOE_DTYPE_BF16)
-    launch_expand<uint16_t>(x, n_tokens, dim, top_k, slot_pos, scores_sorted, routed_input, true, stream);
+    launch_expand<uint16_t>(x, n_tokens, dim, top_k, slot_pos, scores_sorted, routed_input, stream);
   else
-    launch_expand<float>(x, n_tokens, dim, top_k, slot_pos, scores_sorted, routed_input, true, stream);
+    launch_expand<float>(x, n_tokens, dim, top_k, slot_pos, scores_sorted, routed_input, stream);
   return launch_status();
 }
 
@@ -701,9 +757,9 @@ MOE_API int moe_combine_bwd(const void* grad_out, const void* routed_output, con
     if (!slot_pos) return kErrInvalidArgument;
     // plain stores: streaming ones measure 13 % faster alone but 9 % slower in the layer step
     if (dtype == MOE_DTYPE_BF16)
-      launch_expand<uint16_t>(grad_out, n_tokens, dim, top_k, slot_pos, nullptr, grad_routed, false, stream);
+      launch_expand<uint16_t>(grad_out, n_tokens, dim, top_k, slot_pos, nullptr, grad_routed, stream);
     else
-      launch_expand<float>(grad_out, n_tokens, dim, top_k, slot_pos, nullptr, grad_routed, false, stream);
+      launch_expand<float>(grad_out, n_tokens, dim, top_k, slot_pos, nullptr, grad_routed, stream);
   }
   return launch_status();
 }
