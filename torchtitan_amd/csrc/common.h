@@ -134,7 +134,17 @@ __device__ __forceinline__ uint2 pack4(const float (&v)[4]) {
 __device__ __forceinline__ uint2 pack4_mid(const float (&v)[4]) {
   return make_uint2(pack_bf2_mid(v[0], v[1]), pack_bf2_mid(v[2], v[3]));
 }
+__device__ __forceinline__ void unpack4(uint2 w, float (&v)[4]) {
+  v[0] = bf_lo(w.x); v[1] = bf_hi(w.x); v[2] = bf_lo(w.y); v[3] = bf_hi(w.y);
+}
 
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+// a 16-byte load of what is read once: the caches do not keep it
+__device__ __forceinline__ uint4 nt_load(const void* p) {
+  const u32x4_t w = __builtin_nontemporal_load((const u32x4_t*)p);
+  return make_uint4(w.x, w.y, w.z, w.w);
+}
 
 // 16-byte chunks of a bf16 (uint16_t) or fp32 row: 8 or 4 elements widened to
 // fp32, and packed back with the row type's rounding.

@@ -485,7 +485,12 @@ constexpr int kTRows = 128;  // slab rows transposed per pass
 // GATHER: the slab's rows are gathered (RowGather); the indices are loaded two
 // passes ahead of the rows they address and the scale is applied when a pass is
 // consumed, so neither waits behind the row loads in flight.
-template <bool MX, bool ROWS, int COLS, bool GATHER = false, bool ONE = false>
+// NT: weights, read past the caches (this is their last reader in a pass). Experts'
+// forward / backward in us, kept / not kept: MX forward 48 x 768 x 1280 234 -> 220, fp8
+// backward 352 -> 338, 16 x 1536 x 4096 967 -> 940, 64 x 1024 x 2304 825 -> 799 (4096 rows);
+// MX forward of the other two 560 -> 567 and 557 -> 556. Token rows are read again by the
+// next kernel and gain nothing (fp8 backward of 1024 rows 1 % slower).
+template <bool MX, bool ROWS, int COLS, bool GATHER = false, bool ONE = false, bool NT = false>
 __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, int64_t ld, int n_rows, int n_out,
                                              uint8_t* __restrict__ out, int64_t ldo, uint8_t* __restrict__ sc,
                                              int64_t sc_b, int64_t sc_k, const float* s_col, uint32_t* s_tile,
@@ -529,7 +534,9 @@ __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, 
         v[i] = *(const uint4*)(gather.src + (in ? ix[i] : 0) * gather.ld + ch * 8);
         if (gather.scale) sv[i] = gather.scale[clamp_row(a0 + r)];
       } else {
-        v[i] = *(const uint4*)(base + (int64_t)clamp_row(a0 + r) * ld + ch * 8);
+        const uint16_t* row = base + (int64_t)clamp_row(a0 + r) * ld + ch * 8;
+        if constexpr (NT) v[i] = nt_load(row);
+        else v[i] = *(const uint4*)row;
       }
     }
   };
@@ -686,7 +693,7 @@ __global__ __launch_bounds__(4 * COLS) void quant_cols_t_kernel(const uint16_t* 
   }
   __syncthreads();
   const int n = ONE ? min(kTRows, A - a0) : A;
-  slab_t_quant<false, false, COLS, false, ONE>(base + (int64_t)a0 * B, B, n, n, q + e * q_estride + b0 * q_ld + a0, q_ld, nullptr, 0,
+  slab_t_quant<false, false, COLS, false, ONE, true>(base + (int64_t)a0 * B, B, n, n, q + e * q_estride + b0 * q_ld + a0, q_ld, nullptr, 0,
                                    0, s_amax, s_tile);
 }
 
@@ -867,7 +874,7 @@ __global__ __launch_bounds__(4 * COLS) void mx_quant_cols_t_kernel(const uint16_
   const int nb = B / COLS, nch = (A + kTRows - 1) / kTRows;
   const int64_t e = blockIdx.x / (nb * nch);
   const int b0 = (blockIdx.x / nch % nb) * COLS, a0 = blockIdx.x % nch * kTRows, n = min(kTRows, A - a0);
-  slab_t_quant<true, false, COLS, false, true>(x + (e * A + a0) * (int64_t)B + b0, B, n, n, q + e * q_estride + b0 * q_ld + a0, q_ld,
+  slab_t_quant<true, false, COLS, false, true, true>(x + (e * A + a0) * (int64_t)B + b0, B, n, n, q + e * q_estride + b0 * q_ld + a0, q_ld,
                             s + e * s_estride + b0 * s_ld + a0 / kMxBlock, s_ld, 1, nullptr, s_tile);
 }
 
@@ -884,7 +891,7 @@ __global__ __launch_bounds__(4 * COLS) void mx_dual_cols_kernel(const uint16_t* 
   const int64_t e = blockIdx.x / (nb * nch);
   const int b0 = (blockIdx.x / nch % nb) * COLS, a0 = blockIdx.x % nch * kTRows, n = min(kTRows, A - a0);
   const int64_t row0 = e * A + a0;  // the chunk's first row in the [E A, B] view
-  slab_t_quant<true, true, COLS, false, true>(x + row0 * B + b0, B, n, n, q + e * q_estride + b0 * q_ld + a0, q_ld,
+  slab_t_quant<true, true, COLS, false, true, true>(x + row0 * B + b0, B, n, n, q + e * q_estride + b0 * q_ld + a0, q_ld,
                            s + e * s_estride + b0 * s_ld + a0 / kMxBlock, s_ld, 1, nullptr, s_tile, qr + row0 * B + b0, B,
                            sr + row0 * (B / kMxBlock) + b0 / kMxBlock, B / kMxBlock);
 }
@@ -1394,14 +1401,22 @@ __global__ __launch_bounds__(NW * 64, OCC) void fp8_gemm_kernel(Params p) {
               float gv[4], uv[4], hv[4];
 #pragma unroll
               for (int q = 0; q < 4; ++q) {
-                gv[q] = round_bf(MX ? acc[i][2 * jj][q] : (acc[i][2 * jj][q] * sx) * p.sq[e64 * H + hc + q]);
-                uv[q] = round_bf(MX ? acc[i][2 * jj + 1][q] : (acc[i][2 * jj + 1][q] * sx) * p.sq2[e64 * H + hc + q]);
-                // the division: the reciprocal form, chosen per four columns, measured
-                // slower in this epilogue (fp8 1.67 -> 1.69 ms, MX 1.73 -> 1.74 ms)
-                hv[q] = round_bf(silu_sig<false>(gv[q], silu_den(gv[q])).silu) * uv[q];
+                gv[q] = MX ? acc[i][2 * jj][q] : (acc[i][2 * jj][q] * sx) * p.sq[e64 * H + hc + q];
+                uv[q] = MX ? acc[i][2 * jj + 1][q] : (acc[i][2 * jj + 1][q] * sx) * p.sq2[e64 * H + hc + q];
               }
+              // each rounding once, in pairs; those that are not stored keep any NaN (with
+              // the dgu and dx epilogues: experts' forward 1 to 2.5 % faster)
               pg[h2] = pack4(gv);
               pu[h2] = pack4(uv);
+              unpack4(pg[h2], gv);
+              unpack4(pu[h2], uv);
+              // the division: the reciprocal form, chosen per four columns, measured
+              // slower in this epilogue (fp8 1.67 -> 1.69 ms, MX 1.73 -> 1.74 ms)
+#pragma unroll
+              for (int q = 0; q < 4; ++q) hv[q] = silu_sig<false>(gv[q], silu_den(gv[q])).silu;
+              unpack4(pack4_mid(hv), hv);
+#pragma unroll
+              for (int q = 0; q < 4; ++q) hv[q] = hv[q] * uv[q];
               ph[h2] = pack4(hv);
             }
             const int64_t off = (int64_t)r * H + nt * (BN / 2) + wn * (WN / 2) + jp * 32 + g8;
@@ -1448,10 +1463,11 @@ __global__ __launch_bounds__(NW * 64, OCC) void fp8_gemm_kernel(Params p) {
                 uint2 pw;
                 if constexpr (kBatchPark) pw = pws[j];
                 else pw = *(const uint2*)(p.o0 + (int64_t)r * D + n);
-                v[0] = bf_lo(pw.x) + round_bf(v[0]);
-                v[1] = bf_hi(pw.x) + round_bf(v[1]);
-                v[2] = bf_lo(pw.y) + round_bf(v[2]);
-                v[3] = bf_hi(pw.y) + round_bf(v[3]);
+                unpack4(pack4_mid(v), v);
+                v[0] = bf_lo(pw.x) + v[0];
+                v[1] = bf_hi(pw.x) + v[1];
+                v[2] = bf_lo(pw.y) + v[2];
+                v[3] = bf_hi(pw.y) + v[3];
               }
               pv[h2] = pack4(v);
             }
@@ -1505,12 +1521,13 @@ __global__ __launch_bounds__(NW * 64, OCC) void fp8_gemm_kernel(Params p) {
                     f[0] = silu_sig<false>(gv[q], d0);
                     f[1] = silu_sig<false>(gv[q + 1], d1);
                   }
+                  const uint32_t dhw = pack_bf2_mid(acc[i][j][q], acc[i][j][q + 1]);
+                  const uint32_t slw = pack_bf2_mid(f[0].silu, f[1].silu);
+                  const uint32_t dsw = pack_bf2_mid(bf_lo(dhw) * uv[q], bf_hi(dhw) * uv[q + 1]);
 #pragma unroll
                   for (int t = 0; t < 2; ++t) {
-                    const float dh = round_bf(acc[i][j][q + t]);
-                    const float sl = round_bf(f[t].silu);
-                    const float dsl = round_bf(dh * uv[q + t]);
-                    du[q + t] = dh * sl;
+                    const float dsl = t ? bf_hi(dsw) : bf_lo(dsw);
+                    du[q + t] = t ? bf_hi(dhw) * bf_hi(slw) : bf_lo(dhw) * bf_lo(slw);
                     const float sg = f[t].sig;
                     dg[q + t] = dsl * sg * (1.0f + gv[q + t] * (1.0f - sg));
                   }
@@ -1520,13 +1537,17 @@ __global__ __launch_bounds__(NW * 64, OCC) void fp8_gemm_kernel(Params p) {
                 // epilogue, and the reciprocal form's branch spilled it or, per four
                 // columns, made it slower (1.33 -> 1.38 ms)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                  const float dh = round_bf((acc[i][j][q] * sp) * sq4[q]);
-                  const float sl = round_bf(gv[q] / (1.0f + expf(-gv[q])));
-                  const float dsl = round_bf(dh * uv[q]);
-                  du[q] = dh * sl;
-                  const float sg = 1.0f / (1.0f + expf(-gv[q]));
-                  dg[q] = dsl * sg * (1.0f + gv[q] * (1.0f - sg));
+                for (int q = 0; q < 4; q += 2) {
+                  const uint32_t dhw = pack_bf2_mid((acc[i][j][q] * sp) * sq4[q], (acc[i][j][q + 1] * sp) * sq4[q + 1]);
+                  const uint32_t slw = pack_bf2_mid(gv[q] / (1.0f + expf(-gv[q])), gv[q + 1] / (1.0f + expf(-gv[q + 1])));
+                  const uint32_t dsw = pack_bf2_mid(bf_lo(dhw) * uv[q], bf_hi(dhw) * uv[q + 1]);
+#pragma unroll
+                  for (int t = 0; t < 2; ++t) {
+                    const float dsl = t ? bf_hi(dsw) : bf_lo(dsw);
+                    du[q + t] = t ? bf_hi(dhw) * bf_hi(slw) : bf_lo(dhw) * bf_lo(slw);
+                    const float sg = 1.0f / (1.0f + expf(-gv[q + t]));
+                    dg[q + t] = dsl * sg * (1.0f + gv[q + t] * (1.0f - sg));
+                  }
                 }
               }
               pdg[h2] = pack4(dg);

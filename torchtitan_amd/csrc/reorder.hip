@@ -240,12 +240,6 @@ __global__ __launch_bounds__(256) void scatter_kernel(ScatterParams p) {
 // 16-byte chunks (8 bf16 or 4 fp32); arithmetic is fp32 and results are
 // rounded to the row type once, as torch's elementwise ops on that dtype do.
 // ---------------------------------------------------------------------------
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ uint4 nt_load(const void* p) {
-  const u32x4_t w = __builtin_nontemporal_load((const u32x4_t*)p);
-  return make_uint4(w.x, w.y, w.z, w.w);
-}
 
 template <typename T>
 __device__ __forceinline__ uint4 scale_chunk(uint4 v, float s) {
