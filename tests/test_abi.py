@@ -88,6 +88,24 @@ def test_host_side_validation_returns_status_codes(lib):
     assert lib.moe_swiglu_pointwise_f32(null, null, null, 0, null) == 0
 
 
+def test_fp32_experts_take_no_rows(lib):
+    """No rows: every row entry point of the fp32 experts is a no-op that takes the null
+    data pointers of empty tensors; with rows the null tensors are refused. (bwd_dw_all
+    still launches without rows: it clears the weight gradients.)"""
+    null = None
+    some = ctypes.create_string_buffer(64)  # counts: read on the device only
+    for n_rows, want in ((0, 0), (1, -1)):
+        assert lib.moe_zero_rows_past_f32(some, n_rows, 2, null, 64, null, 64, null, 64, null, 64, null) == want
+        assert lib.moe_grouped_gemm_f32_gate_up(null, null, null, some, n_rows, 2, 64, 64, null, null, null, null) == want
+        assert lib.moe_grouped_gemm_f32_down(null, null, some, n_rows, 2, 64, 64, null, null) == want
+        assert lib.moe_grouped_gemm_f32_bwd_dgu(null, null, null, null, some, n_rows, 2, 64, 64, null, null, null) == want
+        assert lib.moe_grouped_gemm_f32_bwd_dx(null, null, null, null, some, n_rows, 2, 64, 64, null, null) == want
+    # what is wrong without rows too
+    assert lib.moe_zero_rows_past_f32(null, 0, 2, null, 64, null, 0, null, 0, null, 0, null) == -1
+    assert lib.moe_zero_rows_past_f32(some, 0, 0, null, 64, null, 0, null, 0, null, 0, null) == -1
+    assert lib.moe_zero_rows_past_f32(some, 0, 2, null, -1, null, 0, null, 0, null, 0, null) == -1
+
+
 def test_status_codes_map_to_exceptions():
     from torchtitan_amd import _lib
 

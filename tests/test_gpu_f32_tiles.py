@@ -63,3 +63,34 @@ def test_f32_tiles(dev, name, shift):
         assert err <= TOL, (what, err)
     for t in (y, g, u, hh, got[0]):
         assert not t[rows - rest:].any(), "rows past the counts are zero"
+
+
+def test_f32_no_rows(dev):
+    """No rows at all (x of zero rows, counts all zero): empty results and zero weight
+    gradients, through the op and through GroupedExperts on the per-expert path, which
+    cuts x to the rows that the counts cover."""
+    from torchtitan_amd import GroupedExperts, ops
+
+    d, h, e = 64, 128, 3
+    banner("fp32 experts without rows")
+    cnt = torch.zeros(e, dtype=torch.int64, device=dev)
+    x = torch.empty(0, d, device=dev, requires_grad=True)
+    ws = [torch.randn(*s, device=dev, requires_grad=True) for s in ((e, h, d), (e, d, h), (e, h, d))]
+    y, g, u, hh = ops.grouped_swiglu_f32(x, *ws, cnt)
+    assert y.shape == (0, d) and g.shape == u.shape == hh.shape == (0, h)
+    got = torch.autograd.grad(y, [x, *ws], torch.empty_like(y))
+    assert got[0].shape == (0, d)
+    for w, gw in zip(ws, got[1:]):
+        assert torch.equal(gw, torch.zeros_like(w))
+
+    experts = GroupedExperts.Config(dim=d, hidden_dim=h, num_experts=e, use_grouped_mm=False).build().to(dev)
+    with torch.no_grad():
+        for p in experts.parameters():
+            p.normal_()
+    for rows in (0, 70):  # 70: rows that no count covers
+        x = torch.randn(rows, d, device=dev, requires_grad=True)
+        y = experts(x, cnt)
+        assert y.shape == (0, d)
+        got = torch.autograd.grad(y, [x, *experts.parameters()], torch.empty_like(y))
+        for t, gt in zip([x, *experts.parameters()], got):
+            assert torch.equal(gt, torch.zeros_like(t))

@@ -519,8 +519,8 @@ MOE_API int moe_zero_rows_past_f32(const int64_t* counts, int64_t n_rows, int32_
                                    hipStream_t stream) {
   if (n_rows < 0 || n_experts < 1 || n_experts > kMaxE || !counts) return kErrInvalidArgument;
   if (cols0 < 0 || cols1 < 0 || cols2 < 0 || cols3 < 0) return kErrInvalidArgument;
+  if (n_rows == 0) return kOk;  // (empty tensors have null pointers)
   if ((cols0 && !t0) || (cols1 && !t1) || (cols2 && !t2) || (cols3 && !t3)) return kErrInvalidArgument;
-  if (n_rows == 0) return kOk;
   const ZeroParams p{counts, n_rows, n_experts, {t0, t1, t2, t3}, {cols0, cols1, cols2, cols3}};
   hipLaunchKernelGGL(zero_rest_kernel, dim3(64), dim3(256), 0, stream, p);
   return launch_status();
