@@ -105,14 +105,24 @@ __device__ __forceinline__ void scan_counts(const int64_t* counts, int64_t R, in
   }
 }
 
-// The expert and 64-row tile of workgroup tile `bx`; e = -1 past the last tile. Every
-// thread of the block must call it.
-__device__ __forceinline__ void find_tile(const Params& p, int bx, int* s_tmp, int* s_out, int& e, Seg& seg, int& mt) {
+// This workgroup's tile: the expert, its 64 rows mt and 64 columns nt of the ntn; e = -1
+// where there is none. Workgroup b runs on XCD b % 8, and each XCD takes an eighth of the
+// tiles, neighbouring ones (they share an operand in its L2): of the tiles that the counts
+// make, not of the grid, which is sized for every row and the worst raggedness. An order over
+// the grid left XCDs idle: with 8192 of 65536 rows in use (8 experts, dim 512, hidden 1024)
+// every tile was on one, gate_up 1154 us, now 193; with all of 8192 rows in use (dim 256,
+// hidden 512) the surplus was all on one, forward 92 -> 77 us, backward 163 -> 140.
+// Every thread of the block must call it.
+__device__ __forceinline__ void find_tile(const Params& p, int ntn, int* s_tmp, int* s_out, int& e, Seg& seg, int& mt,
+                                          int& nt) {
   int cnt[4], st[4], tiles[4], tst[4];
   scan_counts(p.counts, p.R, p.E, s_tmp, st, cnt);
 #pragma unroll
   for (int i = 0; i < 4; ++i) tiles[i] = (cnt[i] + BM - 1) / BM;
   const int total = block_exclusive_scan4(tiles, tst, s_tmp);
+  const int b = blockIdx.x, eighth = (total * ntn + 7) / 8, t = (b & 7) * eighth + (b >> 3);
+  const int bx = (b >> 3) < eighth ? t / ntn : total;
+  nt = t % ntn;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int ee = threadIdx.x * 4 + i;
@@ -167,12 +177,6 @@ __device__ __forceinline__ f32x2_t read_col2(const float* tile, int lane, int w,
   return *(const f32x2_t*)(tile + k * 64 + ((c ^ ((g & 1) << 3)) << 2) + 2 * (lane & 1));
 }
 
-// Consecutive workgroups of one XCD take neighbouring tiles (they share an operand in its L2).
-__device__ __forceinline__ int xcd_order() {
-  const int G = gridDim.x, b = blockIdx.x;
-  return G % 8 == 0 ? (b & 7) * (G >> 3) + (b >> 3) : b;
-}
-
 // Row-grouped modes: 64 rows of one expert x 64 output columns. Waves: 32 x 32 each where
 // the weights are k-contiguous (gate_up, down), 16 x 64 where they are k-major (dgu, dx).
 template <int MODE, bool ALIGNED>
@@ -185,11 +189,10 @@ __global__ __launch_bounds__(512, MODE == kGateUp ? 6 : 8) void rows_kernel(Para
   __shared__ int s_tmp[8];
   __shared__ int s_out[4];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ntn = p.N / BN, t = xcd_order();
-  int e, mt;
+  int e, mt, nt;
   Seg seg;
-  find_tile(p, t / ntn, s_tmp, s_out, e, seg, mt);
-  const int n0 = (t % ntn) * BN;
+  find_tile(p, p.N / BN, s_tmp, s_out, e, seg, mt, nt);
+  const int n0 = nt * BN;
   if (e < 0) return;  // past the last tile
   const int64_t row0 = (int64_t)seg.start + (int64_t)mt * BM;
   const int nrows = min(BM, seg.count - mt * BM);
@@ -421,8 +424,8 @@ inline bool aligned16(const void* a, const void* b, const void* c, const void* d
 template <int MODE>
 int launch_rows(const Params& p, hipStream_t stream) {
   if (p.R == 0) return kOk;
-  // >= sum over experts of ceil(count / 64), and as many more as 64-row tiles past the segments
-  const int64_t gx = (p.R + BM - 1) / BM + p.E, grid = gx * (p.N / BN);
+  // >= sum over experts of ceil(count / 64), times the column tiles; whole eighths (find_tile)
+  const int64_t gx = (p.R + BM - 1) / BM + p.E, grid = (gx * (p.N / BN) + 7) / 8 * 8;
   if (grid > 0x7fffffff) return kErrUnsupportedShape;
   const dim3 blocks((unsigned)grid), threads(512);
   if (aligned16(p.a, p.a2, p.b, p.b2)) hipLaunchKernelGGL((rows_kernel<MODE, true>), blocks, threads, 0, stream, p);
