@@ -169,6 +169,22 @@ def test_f32_zero_rows_past(dev, cols, shift, used):
         assert torch.equal(b, want), c
 
 
+@pytest.mark.parametrize("experts", [600, 1023])
+def test_f32_zero_rows_past_sum_of_counts_in_64_bits(dev, experts):
+    """Counts of more rows than there are cover every row: nothing is cleared, also where
+    their sum is past 32 bits: E (2^22 + 2^13) as an int is negative for 600 experts and a
+    little less than the rows for 1023."""
+    from torchtitan_amd import _lib
+
+    banner(f"fp32 rows past the counts, {experts} counts of all rows")
+    rows = (1 << 22) + (1 << 13)
+    cnt = torch.full((experts,), 1 << 40, dtype=torch.int64, device=dev)
+    t = torch.ones(rows, device=dev)
+    _lib.call("moe_zero_rows_past_f32", cnt.data_ptr(), rows, experts, t.data_ptr(), 1, None, 0, None, 0, None, 0,
+              torch.cuda.current_stream().cuda_stream)
+    assert bool((t == 1).all())
+
+
 def test_f32_zero_rows_past_speed(dev):
     """Clearing many rows keeps about the pace of torch's fill (1.05 of its time as measured;
     4-byte stores of 64 blocks took 2.8 times as long)."""

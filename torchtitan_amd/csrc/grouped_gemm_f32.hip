@@ -401,15 +401,21 @@ struct ZeroParams {
   int64_t cols[4];
 };
 __global__ __launch_bounds__(256) void zero_rest_kernel(ZeroParams p) {
-  __shared__ int s_tmp[8];
-  int cnt[4], st[4];
+  // in 64 bits: counts that are all past R sum up to E R, which would wrap an int and put the
+  // first cleared row before the tensor
+  __shared__ int64_t s_sum[4];
+  int64_t total = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int ee = threadIdx.x * 4 + i;
     const int64_t c = ee < p.E ? p.counts[ee] : 0;
-    cnt[i] = c < 0 ? 0 : (int)(c > p.R ? p.R : c);
+    total += c < 0 ? 0 : (c > p.R ? p.R : c);
   }
-  const int64_t total = block_exclusive_scan4(cnt, st, s_tmp);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off);
+  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = total;
+  __syncthreads();
+  total = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
   if (total >= p.R) return;
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
 #pragma unroll
