@@ -212,3 +212,96 @@ def test_f32_zero_rows_past_speed(dev):
     rest = fastest(lambda: _lib.call("moe_zero_rows_past_f32", cnt.data_ptr(), rows, 1, *args, st))
     print(f"fill {fill * 1e3:.0f} us, rows past the counts {rest * 1e3:.0f} us", flush=True)
     assert rest < 1.6 * fill
+
+
+def test_f32_grid_slices(dev):
+    """Grids of a little more than one slice of 65536 workgroups, every entry point:
+    the same result as its parts launched alone (narrower weights, or fewer experts), whose
+    grids are one slice; the sums are the same ones in the same order."""
+    from torchtitan_amd import _lib
+
+    banner("fp32 grids of two slices")
+    gen = torch.Generator(device=dev).manual_seed(5)
+    st = torch.cuda.current_stream().cuda_stream
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=gen, device=dev)
+
+    def run(name, ins, dims, outs):
+        _lib.call("moe_grouped_gemm_f32_" + name, *(t.data_ptr() for t in ins), *dims,
+                  *(t.data_ptr() for t in outs), st)
+        return outs
+
+    rows, wide, k, e = 2112, 131072, 64, 2  # (33 + 2) x 2048 tiles
+    cnt = torch.tensor([1000, 1112], dtype=torch.int64, device=dev)
+    a, a2, w, w3 = rnd(rows, k), rnd(rows, k), rnd(e, wide, k), rnd(e, wide, k)
+    gw, uw = rnd(rows, wide), rnd(rows, wide)
+    half = wide // 2
+    cut = [(lambda t, i=i: t[..., i * half:(i + 1) * half].contiguous()) for i in range(2)]
+    cute = [(lambda t, i=i: t[:, i * half:(i + 1) * half].contiguous()) for i in range(2)]
+
+    def new(n, cols):
+        return [torch.full((rows, cols), float("nan"), device=dev) for _ in range(n)]
+
+    got = run("gate_up", [a, w, w3, cnt], (rows, e, k, wide), new(3, wide))
+    for i in range(2):
+        part = run("gate_up", [a, cute[i](w), cute[i](w3), cnt], (rows, e, k, half), new(3, half))
+        assert all(torch.equal(cut[i](x), y) for x, y in zip(got, part))
+    got = run("down", [a, w, cnt], (rows, e, wide, k), new(1, wide))
+    for i in range(2):
+        assert torch.equal(cut[i](got[0]), run("down", [a, cute[i](w), cnt], (rows, e, half, k), new(1, half))[0])
+    wt, w3t = w.view(e, k, wide), w3.view(e, k, wide)
+    got = run("bwd_dgu", [a, wt, gw, uw, cnt], (rows, e, k, wide), new(2, wide))
+    for i in range(2):
+        part = run("bwd_dgu", [a, cut[i](wt), cut[i](gw), cut[i](uw), cnt], (rows, e, k, half), new(2, half))
+        assert all(torch.equal(cut[i](x), y) for x, y in zip(got, part))
+    got = run("bwd_dx", [a, a2, wt, w3t, cnt], (rows, e, wide, k), new(1, wide))
+    for i in range(2):
+        part = run("bwd_dx", [a, a2, cut[i](wt), cut[i](w3t), cnt], (rows, e, half, k), new(1, half))
+        assert torch.equal(cut[i](got[0]), part[0])
+    del got, part, w, w3, wt, w3t, gw, uw
+
+    m, n, e, rows = 2048, 4096, 33, 660  # 33 x 2048 tiles a weight
+    cnt = torch.full((e,), rows // e, dtype=torch.int64, device=dev)
+    dg, du, h, x, dy = rnd(rows, n), rnd(rows, n), rnd(rows, n), rnd(rows, m), rnd(rows, m)
+
+    def all3(lo, hi):
+        s = slice(lo * rows // e, hi * rows // e)
+        outs = [torch.full((hi - lo, *d), float("nan"), device=dev) for d in ((n, m), (n, m), (m, n))]
+        ins = [t[s].contiguous() for t in (dg, du, dy, x, h)]
+        run("bwd_dw_all", [*ins, cnt[lo:hi].contiguous()], ((hi - lo) * rows // e, hi - lo, m, n), outs)
+        one = torch.full((hi - lo, n, m), float("nan"), device=dev)
+        run("bwd_dw", [ins[0], ins[3], cnt[lo:hi].contiguous()], ((hi - lo) * rows // e, hi - lo, n, m), [one])
+        return [*outs, one]
+
+    got = all3(0, e)
+    for lo, hi in ((0, 8), (8, 16), (16, 24), (24, 33)):
+        assert all(torch.equal(x[lo:hi], y) for x, y in zip(got, all3(lo, hi)))
+
+
+def test_f32_more_than_2_32_threads(dev):
+    """8.4 million output rows of 4096 columns (137 GB) are 2^23 tiles and more, 2^32 threads
+    of one launch: rows of the first, the last and of tiles between against 64 bits."""
+    from torchtitan_amd import _lib
+
+    d, h, rows = 4096, 64, (1 << 23) + 64
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < rows * (d + h) * 4 + (8 << 30):
+        pytest.skip("needs 148 GB of free device memory")
+    banner("fp32 down, 2^23 + 64 rows of 4096")
+    gen = torch.Generator(device=dev).manual_seed(6)
+    x = torch.randn(rows, h, generator=gen, device=dev)
+    w2 = torch.randn(1, d, h, generator=gen, device=dev)
+    cnt = torch.tensor([rows], dtype=torch.int64, device=dev)
+    y = torch.empty(rows, d, device=dev)
+    try:
+        y[-64:].fill_(float("nan"))
+        _lib.call("moe_grouped_gemm_f32_down", x.data_ptr(), w2.data_ptr(), cnt.data_ptr(), rows, 1, d, h,
+                  y.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        for r in (0, 1 << 20, (1 << 22) - 64, 1 << 22, 1 << 23):
+            want = x[r:r + 64].double() @ w2[0].double().t()
+            err = (y[r:r + 64].double() - want).abs().max().item() / want.abs().max().item()
+            assert err <= TOL, (r, err)
+    finally:
+        del y, x
+        torch.cuda.empty_cache()

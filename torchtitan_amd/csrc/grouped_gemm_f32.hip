@@ -84,6 +84,15 @@ __device__ __forceinline__ void copy16(const float* g, uint32_t lds) {
 }
 __device__ __forceinline__ uint32_t lds_addr(float* p) { return (uint32_t)(size_t)((LDSP float*)p); }
 
+// Grids have up to 2^31 workgroups, more than a launch allows in x (under 2^32 threads):
+// slices of whole eighths in x (a multiple of the XCDs), as many as needed in y.
+constexpr int kSlice = 1 << 16;
+inline dim3 sliced(int64_t grid) {
+  return grid <= kSlice ? dim3((unsigned)grid) : dim3(kSlice, (unsigned)((grid + kSlice - 1) / kSlice));
+}
+constexpr int64_t kMaxGrid = 0x7fffffff - kSlice;
+__device__ __forceinline__ int workgroup() { return (int)(blockIdx.y * gridDim.x + blockIdx.x); }
+
 // Expert segments: rows [start, start + count) clamped to R.
 struct Seg { int start, count; };
 
@@ -120,7 +129,7 @@ __device__ __forceinline__ void find_tile(const Params& p, int ntn, int* s_tmp, 
 #pragma unroll
   for (int i = 0; i < 4; ++i) tiles[i] = (cnt[i] + BM - 1) / BM;
   const int total = block_exclusive_scan4(tiles, tst, s_tmp);
-  const int b = blockIdx.x, eighth = (total * ntn + 7) / 8, t = (b & 7) * eighth + (b >> 3);
+  const int b = workgroup(), eighth = (total * ntn + 7) / 8, t = (b & 7) * eighth + (b >> 3);
   const int bx = (b >> 3) < eighth ? t / ntn : total;
   nt = t % ntn;
 #pragma unroll
@@ -315,6 +324,7 @@ struct DwParams {
   int64_t R;
   int E;
   int per_e;  // tiles of one expert, the same in every job: M N / 64^2
+  int tiles;  // of all jobs
   DwJob job[3];
 };
 
@@ -330,7 +340,8 @@ __global__ __launch_bounds__(256, 4) void dw_kernel(DwParams p) {
   // idle where the experts' row counts differ. The jobs start at experts a third apart:
   // a CU's workgroups, a chip apart in the grid, would otherwise all belong to the same
   // heavy expert.
-  const int q = p.per_e % 8 == 0 ? p.per_e >> 3 : 0, b = blockIdx.x;
+  const int q = p.per_e % 8 == 0 ? p.per_e >> 3 : 0, b = workgroup();
+  if (b >= p.tiles) return;
   const int group = q ? (b >> 3) / q : b / p.per_e;
   const int t = q ? (b & 7) * q + (b >> 3) % q : b % p.per_e;
   const int ji = group / p.E, e = (group + ji * ((p.E + 2) / 3)) % p.E;
@@ -443,8 +454,8 @@ int launch_rows(const Params& p, hipStream_t stream) {
   if (p.R == 0) return kOk;
   // >= sum over experts of ceil(count / 64), times the column tiles; whole eighths (find_tile)
   const int64_t gx = (p.R + BM - 1) / BM + p.E, grid = (gx * (p.N / BN) + 7) / 8 * 8;
-  if (grid > 0x7fffffff) return kErrUnsupportedShape;
-  const dim3 blocks((unsigned)grid), threads(512);
+  if (grid > kMaxGrid) return kErrUnsupportedShape;
+  const dim3 blocks = sliced(grid), threads(512);
   if (aligned16(p.a, p.a2, p.b, p.b2)) hipLaunchKernelGGL((rows_kernel<MODE, true>), blocks, threads, 0, stream, p);
   else hipLaunchKernelGGL((rows_kernel<MODE, false>), blocks, threads, 0, stream, p);
   return launch_status();
@@ -452,12 +463,13 @@ int launch_rows(const Params& p, hipStream_t stream) {
 
 int launch_dw(DwParams& p, int jobs, hipStream_t stream) {
   const int64_t per_e = (int64_t)(p.job[0].M / BM) * (p.job[0].N / BN), grid = per_e * p.E * jobs;
-  if (grid > 0x7fffffff) return kErrUnsupportedShape;
+  if (grid > kMaxGrid) return kErrUnsupportedShape;
   p.per_e = (int)per_e;
+  p.tiles = (int)grid;
   bool aligned = true;
   for (int j = 0; j < jobs; ++j) aligned = aligned && aligned16(p.job[j].a, p.job[j].b, nullptr, nullptr);
-  if (aligned) hipLaunchKernelGGL(dw_kernel<true>, dim3((unsigned)grid), dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL(dw_kernel<false>, dim3((unsigned)grid), dim3(256), 0, stream, p);
+  if (aligned) hipLaunchKernelGGL(dw_kernel<true>, sliced(grid), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL(dw_kernel<false>, sliced(grid), dim3(256), 0, stream, p);
   return launch_status();
 }
 
