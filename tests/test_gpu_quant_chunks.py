@@ -106,3 +106,43 @@ def test_weight_chunks(dev, a, b):
     call("moe_fp8_quant_cols_t_amax", ptr(x), ptr(amax), e, a, b, ptr(f[0][0]), a * b, a, ptr(f[0][1]), b, st)
     call("moe_fp8_quant_cols_t", ptr(x), e, a, b, ptr(f[1][0]), a * b, a, ptr(f[1][1]), b, st)
     assert torch.equal(f[0][0], f[1][0]) and torch.equal(f[0][1], f[1][1])
+
+
+def test_token_chunks_more_than_2_32_threads(dev):
+    """8.4 million gathered rows of 16384 columns (137 GB of fp8) are 2^23 blocks and more,
+    2^32 threads of one launch: columns of the first, the last and of slabs between against
+    a small call on the 64 rows that all of them repeat."""
+    from torchtitan_amd._lib import call, ptr
+
+    c, n_src = 16384, 64
+    r = (1 << 23) + n_src
+    rpad = (r + 127) // 128 * 128 + 128
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < c * rpad + (8 << 30):
+        pytest.skip("needs 146 GB of free device memory")
+    banner("fp8 token quantizer, 2^23 + 64 rows of 16384")
+    gen = torch.Generator(device=dev).manual_seed(7)
+    src = torch.randn(n_src, c, generator=gen, device=dev).bfloat16()
+    amax = src.float().abs().amax(0)[None].contiguous()
+    st = torch.cuda.current_stream().cuda_stream
+
+    def quant(rows, padded):
+        idx = torch.arange(rows, device=dev) % n_src
+        counts = torch.tensor([rows], dtype=torch.int64, device=dev)
+        q = torch.empty(c, padded, dtype=torch.uint8, device=dev)
+        s = torch.empty(1, c, device=dev)
+        call("moe_fp8_quant_tokens_t_amax_gather", ptr(src), n_src, ptr(idx), None, ptr(amax), ptr(counts), rows, 1, c,
+             padded, ptr(q), ptr(s), st)
+        return q, s
+
+    want, ws = quant(n_src, 256)
+    q, s = quant(r, rpad)
+    try:
+        assert torch.equal(s, ws)
+        for col in (0, 1, 127, 128, 8191, 8192, c - 129, c - 1):
+            row = q[col, :r].view(-1, n_src)
+            assert bool((row == want[col, :n_src]).all()), col
+            assert not q[col, r:(r + 127) // 128 * 128].any(), col
+    finally:
+        del q
+        torch.cuda.empty_cache()

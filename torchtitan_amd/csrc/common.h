@@ -28,6 +28,16 @@ inline int launch_status() {
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
+// Flat grids of up to 2^31 workgroups, more than a launch takes in x (under 2^32 threads):
+// slices of 65536 (a multiple of the XCDs) in x, as many as needed in y; the last slice
+// has workgroups past the grid.
+constexpr int kSlice = 1 << 16;
+constexpr int64_t kMaxGrid = 0x7fffffff - kSlice;
+inline dim3 sliced(int64_t grid) {
+  return grid <= kSlice ? dim3((unsigned)grid) : dim3(kSlice, (unsigned)((grid + kSlice - 1) / kSlice));
+}
+__device__ __forceinline__ int workgroup() { return (int)(blockIdx.y * gridDim.x + blockIdx.x); }
+
 // ---------------------------------------------------------------------------
 // bf16 <-> fp32. The narrowing conversion is round-to-nearest-even with NaN
 // mapped to the canonical quiet NaN 0x7FC0, which is what torch's bf16 casts do.

@@ -778,9 +778,10 @@ __global__ __launch_bounds__(4 * COLS) void quant_tokens_t_kernel(const uint16_t
   __shared__ GroupChunk s_gc;
   // slab-major: the blocks running together share column slabs (1-4 % faster
   // than expert-major at the Kimi shapes)
-  const int n_chunks = ONE ? (int)(R / kTRows) + E : E;
-  const int c0 = (blockIdx.x / n_chunks) * COLS;
-  int e = blockIdx.x % n_chunks, seg0, pstart, n, off = 0;
+  const int n_chunks = ONE ? (int)(R / kTRows) + E : E, b = workgroup();
+  const int c0 = b / n_chunks * COLS;
+  if (c0 >= C) return;
+  int e = b % n_chunks, seg0, pstart, n, off = 0;
   if constexpr (ONE) {
     const GroupChunk gc = find_chunk(counts, R, E, e, s_tmp, &s_gc);
     if (gc.e < 0) return;
@@ -910,9 +911,10 @@ __global__ __launch_bounds__(4 * COLS) void mx_quant_tokens_t_kernel(const uint1
   __shared__ __attribute__((aligned(16))) uint32_t s_tile[kTRows * (COLS / 2)];
   __shared__ int s_tmp[8];
   __shared__ GroupChunk s_gc;
-  const int n_chunks = (int)(R / kTRows) + E + kTailBlocks;
-  const int c0 = (blockIdx.x / n_chunks) * COLS;  // slab-major: blocks running together share column slabs
-  const GroupChunk gc = find_chunk(counts, R, E, blockIdx.x % n_chunks, s_tmp, &s_gc);
+  const int n_chunks = (int)(R / kTRows) + E + kTailBlocks, b = workgroup();
+  const int c0 = b / n_chunks * COLS;  // slab-major: blocks running together share column slabs
+  if (c0 >= C) return;
+  const GroupChunk gc = find_chunk(counts, R, E, b % n_chunks, s_tmp, &s_gc);
   const int e = gc.e, seg0 = gc.seg0, pstart = gc.pstart, off = gc.off;
   int n = gc.n;
   if ((int64_t)seg0 + n > R) n = (int)(R - seg0 > 0 ? R - seg0 : 0);
@@ -1751,10 +1753,10 @@ static int quant_tokens_t(const uint16_t* x, const float* group_amax, const int6
                          : (one ? quant_tokens_t_kernel<64, true> : quant_tokens_t_kernel<64, false>);
   const int64_t n_blocks = one ? n_rows / kTRows + n_experts : n_experts;
   if (cols % 128 == 0)
-    hipLaunchKernelGGL(k128, dim3((unsigned)(n_blocks * (cols / 128))), dim3(512), 0, stream, x, counts, n_rows, n_experts, cols,
+    hipLaunchKernelGGL(k128, sliced(n_blocks * (cols / 128)), dim3(512), 0, stream, x, counts, n_rows, n_experts, cols,
                        padded_rows, q, scale, group_amax, gather);
   else
-    hipLaunchKernelGGL(k64, dim3((unsigned)(n_blocks * (cols / 64))), dim3(256), 0, stream, x, counts, n_rows, n_experts, cols,
+    hipLaunchKernelGGL(k64, sliced(n_blocks * (cols / 64)), dim3(256), 0, stream, x, counts, n_rows, n_experts, cols,
                        padded_rows, q, scale, group_amax, gather);
   return launch_status();
 }
@@ -2002,11 +2004,11 @@ MOE_API int moe_mxfp8_quant_tokens_t(const uint16_t* x, const int64_t* counts, i
   if (!x || !counts || !q || !scale) return kErrInvalidArgument;
   const int64_t n_blocks = token_blocks(n_rows, n_experts);
   if (cols % 128 == 0)
-    hipLaunchKernelGGL((mx_quant_tokens_t_kernel<false, 128>), dim3((unsigned)(n_blocks * (cols / 128))), dim3(512), 0, stream, x,
+    hipLaunchKernelGGL((mx_quant_tokens_t_kernel<false, 128>), sliced(n_blocks * (cols / 128)), dim3(512), 0, stream, x,
                        counts, n_rows, n_experts, cols, padded_rows, q, scale, (uint8_t*)nullptr, (uint8_t*)nullptr,
                        RowGather{});
   else
-    hipLaunchKernelGGL((mx_quant_tokens_t_kernel<false, 64>), dim3((unsigned)(n_blocks * (cols / 64))), dim3(256), 0, stream, x,
+    hipLaunchKernelGGL((mx_quant_tokens_t_kernel<false, 64>), sliced(n_blocks * (cols / 64)), dim3(256), 0, stream, x,
                        counts, n_rows, n_experts, cols, padded_rows, q, scale, (uint8_t*)nullptr, (uint8_t*)nullptr,
                        RowGather{});
   return launch_status();
@@ -2045,10 +2047,10 @@ static int mx_dual_tokens(const uint16_t* x, RowGather gather, const int64_t* co
   const kernel_t k128 = g ? mx_quant_tokens_t_kernel<true, 128, true> : mx_quant_tokens_t_kernel<true, 128, false>;
   const kernel_t k64 = g ? mx_quant_tokens_t_kernel<true, 64, true> : mx_quant_tokens_t_kernel<true, 64, false>;
   if (cols % 128 == 0)
-    hipLaunchKernelGGL(k128, dim3((unsigned)(n_blocks * (cols / 128))), dim3(512), 0, stream, x, counts, n_rows, n_experts, cols,
+    hipLaunchKernelGGL(k128, sliced(n_blocks * (cols / 128)), dim3(512), 0, stream, x, counts, n_rows, n_experts, cols,
                        padded_rows, q, scale, q_rows, scale_rows, gather);
   else
-    hipLaunchKernelGGL(k64, dim3((unsigned)(n_blocks * (cols / 64))), dim3(256), 0, stream, x, counts, n_rows, n_experts, cols,
+    hipLaunchKernelGGL(k64, sliced(n_blocks * (cols / 64)), dim3(256), 0, stream, x, counts, n_rows, n_experts, cols,
                        padded_rows, q, scale, q_rows, scale_rows, gather);
   return launch_status();
 }

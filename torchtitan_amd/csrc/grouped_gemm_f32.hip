@@ -84,15 +84,6 @@ __device__ __forceinline__ void copy16(const float* g, uint32_t lds) {
 }
 __device__ __forceinline__ uint32_t lds_addr(float* p) { return (uint32_t)(size_t)((LDSP float*)p); }
 
-// Grids have up to 2^31 workgroups, more than a launch allows in x (under 2^32 threads):
-// slices of whole eighths in x (a multiple of the XCDs), as many as needed in y.
-constexpr int kSlice = 1 << 16;
-inline dim3 sliced(int64_t grid) {
-  return grid <= kSlice ? dim3((unsigned)grid) : dim3(kSlice, (unsigned)((grid + kSlice - 1) / kSlice));
-}
-constexpr int64_t kMaxGrid = 0x7fffffff - kSlice;
-__device__ __forceinline__ int workgroup() { return (int)(blockIdx.y * gridDim.x + blockIdx.x); }
-
 // Expert segments: rows [start, start + count) clamped to R.
 struct Seg { int start, count; };
 
