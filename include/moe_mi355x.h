@@ -233,6 +233,14 @@ int moe_grouped_gemm_bwd_dw2(const uint16_t* dy, const uint16_t* h, const int64_
 int moe_swiglu_pointwise_f32(const uint16_t* g, float* silu, float* sigmoid, int64_t n,
                              moe_stream_t stream);
 
+/* No counterpart in the reference; for tests: the tile that a bf16 grouped GEMM launch
+ * takes on a GPU of n_cus compute units, as 10000 rows + 10 columns + workgroups per CU
+ * (128 x 384, one per CU: 1283841). mode 0..5: gate_up, down, bwd_dgu, bwd_dx, bwd_dw13
+ * (gpt-oss: bwd_dw1), bwd_dw2; gptoss != 0: the gpt-oss entry points. A negative status
+ * where the launch would refuse the shape. Nothing is launched. */
+int moe_grouped_gemm_tile(int32_t mode, int32_t gptoss, int64_t n_rows, int32_t n_experts, int32_t dim,
+                          int32_t hidden, int32_t n_cus);
+
 /* ---- fp32 experts: _run_experts_for_loop in the input dtype --------------
  * Replace the per-expert fp32 matmuls of torchtitan/models/common/moe.py:24-50
  * (and their autograd) with one launch per GEMM over all experts: fp32

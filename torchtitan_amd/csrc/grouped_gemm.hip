@@ -976,59 +976,71 @@ static void launch_cfg(const GemmParams& p, int64_t R, hipStream_t stream) {
 // 309; dW 256 / 512 / 8 / 8192 42 -> 24. The weights are read once whatever the tile: with
 // few rows per expert the eight-wave forward tile's three stages of whole 128-byte rows
 // keep more bytes in flight (5.2 -> 6.1 TB/s of weights at two rows per expert).
-static double rounds(double tiles, int per_cu) {
-  const double slots = (double)cu_count() * per_cu;
+enum GemmTile : int {  // rows x columns, workgroups per CU: 10000 rows + 10 columns + workgroups
+  k128x256 = 1282561, k256x256 = 2562561, k128x384 = 1283841, k128x512 = 1285121,
+  k64x256Two = 642562, k128x256Two = 1282562, k128x128Two = 1281282
+};
+static double rounds(double tiles, int slots) {
   return tiles <= slots ? 1.0 : (double)((int64_t)((tiles + slots - 1.0) / slots));
 }
 static double expected_m_tiles(int64_t R, int64_t E, int bm) {
   const double whole = (double)R / bm + 0.5 * (double)E, least = (double)(R < E ? R : E);
   return whole > least ? whole : least;
 }
+static GemmTile pick_tile(int mode, int act, int64_t R, int64_t E, int64_t D, int64_t H, int cus) {
+  auto n_tiles = [](int64_t n, int bn) { return (double)((n + bn - 1) / bn); };
+  const double m256 = expected_m_tiles(R, E, 256), m128 = expected_m_tiles(R, E, 128),
+               m64 = expected_m_tiles(R, E, 64), least = (double)(R < E ? R : E);
+  if (mode == kFwdGateUp || mode == kFwdDown) {
+    const double nt = n_tiles(mode == kFwdGateUp ? 2 * H : D, 256);
+    const double tall = mode == kFwdGateUp && act == kOssGLU ? 1.62 : 1.7;
+    return tall * rounds(m256 * nt, cus) < rounds(m128 * nt, cus) ? k256x256 : k128x256;
+  }
+  if (mode == kBwdDgu) {
+    const double nt = n_tiles(H, 256);
+    const double c_one = rounds(m128 * nt, cus), c_two = 1.74 * rounds(m128 * nt, 2 * cus),
+                 c_low = 1.45 * rounds(m64 * nt, 2 * cus);
+    if (m64 > least && c_low < c_one && c_low < c_two) return k64x256Two;
+    return c_two < c_one ? k128x256Two : k128x256;
+  }
+  if (mode == kBwdDx) {
+    const double c256 = rounds(m128 * n_tiles(D, 256), cus),
+                 c384 = (m128 > least ? 1.45 : 1.55) * rounds(m128 * n_tiles(D, 384), cus),
+                 c512 = act == kOssGLU || D % 512 == 0 ? 1.73 * rounds(m128 * n_tiles(D, 512), cus) : INFINITY,
+                 c_two = 1.95 * rounds(m128 * n_tiles(D, 256), 2 * cus),
+                 c_tall = act == kOssGLU ? 1.62 * rounds(m256 * n_tiles(D, 256), cus) : INFINITY;
+    const double best = fmin(fmin(c256, c384), fmin(fmin(c512, c_tall), c_two));
+    return best == c_tall ? k256x256 : best == c384 ? k128x384 : best == c512 ? k128x512
+           : best == c256 ? k128x256 : k128x256Two;
+  }
+  const int64_t m = mode == kBwdDw13 ? 2 * H : D, n = mode == kBwdDw13 ? D : H;
+  return 2 * E * n_tiles(m, 256) * n_tiles(n, 256) <= cus ? k128x128Two : k256x256;
+}
 
 template <int MODE, int ACT = kSwiGLU>
 static void launch_mode(const GemmParams& p, int64_t R, hipStream_t stream) {
-  auto n_tiles = [](int64_t n, int bn) { return (double)((n + bn - 1) / bn); };
-  const double m256 = expected_m_tiles(R, p.E, 256), m128 = expected_m_tiles(R, p.E, 128),
-               m64 = expected_m_tiles(R, p.E, 64);
+  const GemmTile tile = pick_tile(MODE, ACT, R, p.E, p.D, p.H, cu_count());
   if constexpr (MODE == kFwdGateUp || MODE == kFwdDown) {
-    const double nt = n_tiles(MODE == kFwdGateUp ? 2 * (int64_t)p.H : p.D, 256);
-    const double tall = MODE == kFwdGateUp && ACT == kOssGLU ? 1.62 : 1.7;
-    if (tall * rounds(m256 * nt, 1) < rounds(m128 * nt, 1))
-      launch_cfg<MODE, 8, 4, 4, 8, 2, true, 1, ACT, 64>(p, R, stream);
-    else
-      launch_cfg<MODE, 8, 2, 4, 4, 3, true, 1, ACT, 64>(p, R, stream);
+    if (tile == k256x256) launch_cfg<MODE, 8, 4, 4, 8, 2, true, 1, ACT, 64>(p, R, stream);
+    else launch_cfg<MODE, 8, 2, 4, 4, 3, true, 1, ACT, 64>(p, R, stream);
   } else if constexpr (MODE == kBwdDgu) {
-    const double nt = n_tiles(p.H, 256);
-    const double c_one = rounds(m128 * nt, 1), c_two = 1.74 * rounds(m128 * nt, 2),
-                 c_low = 1.45 * rounds(m64 * nt, 2);
-    const bool several = m64 > (double)(R < p.E ? R : p.E);
-    if (several && c_low < c_one && c_low < c_two) launch_cfg<MODE, 4, 1, 4, 4, 3, true, 2, ACT>(p, R, stream);
-    else if (c_two < c_one) launch_cfg<MODE, 4, 2, 4, 8, 2, true, 2, ACT>(p, R, stream);
+    if (tile == k64x256Two) launch_cfg<MODE, 4, 1, 4, 4, 3, true, 2, ACT>(p, R, stream);
+    else if (tile == k128x256Two) launch_cfg<MODE, 4, 2, 4, 8, 2, true, 2, ACT>(p, R, stream);
     else launch_cfg<MODE, 8, 2, 4, 4, 3, true, 1, ACT>(p, R, stream);
   } else if constexpr (MODE == kBwdDx) {
-    const bool several = m128 > (double)(R < p.E ? R : p.E);
-    const double c256 = rounds(m128 * n_tiles(p.D, 256), 1),
-                 c384 = (several ? 1.45 : 1.55) * rounds(m128 * n_tiles(p.D, 384), 1),
-                 c512 = ACT == kOssGLU || p.D % 512 == 0 ? 1.73 * rounds(m128 * n_tiles(p.D, 512), 1) : INFINITY,
-                 c_two = 1.95 * rounds(m128 * n_tiles(p.D, 256), 2);
-    const double c_tall = ACT == kOssGLU ? 1.62 * rounds(m256 * n_tiles(p.D, 256), 1) : INFINITY;
-    const double best = fmin(fmin(c256, c384), fmin(fmin(c512, c_tall), c_two));
     if constexpr (ACT == kOssGLU) {
-      if (best == c_tall) {
+      if (tile == k256x256) {
         launch_cfg<MODE, 8, 4, 4, 8, 3, false, 1, ACT>(p, R, stream);
         return;
       }
     }
-    if (best == c384) launch_cfg<MODE, 8, 2, 4, 6, 3, false, 1, ACT>(p, R, stream);
-    else if (best == c512) launch_cfg<MODE, 8, 2, 4, 8, 3, false, 1, ACT>(p, R, stream);
-    else if (best == c256) launch_cfg<MODE, 8, 2, 4, 4, 3, false, 1, ACT>(p, R, stream);
+    if (tile == k128x384) launch_cfg<MODE, 8, 2, 4, 6, 3, false, 1, ACT>(p, R, stream);
+    else if (tile == k128x512) launch_cfg<MODE, 8, 2, 4, 8, 3, false, 1, ACT>(p, R, stream);
+    else if (tile == k128x256) launch_cfg<MODE, 8, 2, 4, 4, 3, false, 1, ACT>(p, R, stream);
     else launch_cfg<MODE, 4, 2, 4, 8, 2, false, 2, ACT>(p, R, stream);
   } else {
-    const int64_t m = MODE == kBwdDw13 ? 2 * (int64_t)p.H : p.D, n = MODE == kBwdDw13 ? p.D : p.H;
-    if (2 * p.E * n_tiles(m, 256) * n_tiles(n, 256) <= cu_count())
-      launch_cfg<MODE, 4, 2, 4, 4, 3, false, 2, kSwiGLU>(p, R, stream);
-    else
-      launch_cfg<MODE, 8, 4, 4, 8, 3, false, 1, kSwiGLU>(p, R, stream);
+    if (tile == k128x128Two) launch_cfg<MODE, 4, 2, 4, 4, 3, false, 2, kSwiGLU>(p, R, stream);
+    else launch_cfg<MODE, 8, 4, 4, 8, 3, false, 1, kSwiGLU>(p, R, stream);
   }
 }
 
@@ -1165,6 +1177,13 @@ MOE_API int moe_swiglu_pointwise_f32(const uint16_t* g, float* silu, float* sigm
   if (blocks > 0x7fffffff) return kErrInvalidArgument;
   swiglu_pointwise_kernel<<<(unsigned)blocks, 256, 0, stream>>>(g, silu, sigmoid, n);
   return launch_status();
+}
+
+MOE_API int moe_grouped_gemm_tile(int32_t mode, int32_t gptoss, int64_t n_rows, int32_t n_experts, int32_t dim,
+                                  int32_t hidden, int32_t n_cus) {
+  if (mode < kFwdGateUp || mode > kBwdDw2 || n_cus < 1) return kErrInvalidArgument;
+  const int st = check_gemm_shape(n_rows, n_experts, dim, hidden);
+  return st ? st : pick_tile(mode, gptoss ? kOssGLU : kSwiGLU, n_rows, n_experts, dim, hidden, n_cus);
 }
 
 MOE_API int moe_grouped_swiglu_fwd(const uint16_t* x, const uint16_t* w1, const uint16_t* w2,
