@@ -76,6 +76,33 @@ def test_token_chunks(dev, name):
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
 
 
+def test_token_chunks_counts_past_the_rows(dev):
+    """Counts that sum up to twice the rows make more chunks than the launch has blocks:
+    the columns past the last group, whose rows all lie past R, are still cleared, and the
+    first group's bytes are those of its rows alone."""
+    from torchtitan_amd import _lib
+    from torchtitan_amd._lib import call, ptr
+
+    r, c = 1536, 128
+    banner("MX token quantizer, counts past the rows")
+    gen = torch.Generator(device=dev).manual_seed(8)
+    x = torch.randn(r, c, generator=gen, device=dev).bfloat16()
+    st = torch.cuda.current_stream().cuda_stream
+
+    def quant(groups):
+        e = len(groups)
+        counts = torch.tensor(groups, dtype=torch.int64, device=dev)
+        rpad = int(_lib.lib().moe_mxfp8_padded_rows(r, e))
+        q, s = (torch.full(d, 0xA5, dtype=torch.uint8, device=dev) for d in ((c, rpad), (rpad // 32, c)))
+        call("moe_mxfp8_quant_tokens_t", ptr(x), ptr(counts), r, e, c, rpad, ptr(q), ptr(s), st)
+        return q, s
+
+    q, s = quant([r, r])
+    want_q, want_s = quant([r])
+    assert torch.equal(q[:, :r], want_q[:, :r]) and torch.equal(s[:r // 32], want_s[:r // 32])
+    assert q.shape[1] > r and not q[:, r:].any() and not s[r // 32:].any()
+
+
 @pytest.mark.parametrize("a,b", [(32, 64), (128, 128), (160, 192), (352, 128)])
 def test_weight_chunks(dev, a, b):
     from torchtitan_amd._lib import call, ptr

@@ -699,8 +699,8 @@ __global__ __launch_bounds__(4 * COLS) void quant_cols_t_kernel(const uint16_t* 
 
 // The 128 rows of one token group that a block transposes: rows off .. of group e, which
 // starts at row seg0 and at pstart of the padded layout (its 128-row chunks before it times
-// 128) and has n rows. Past the last chunk e is -1, off counts the chunks past it and seg0,
-// pstart, n describe the last group. Every thread of the block calls it. Up to 256 groups
+// 128) and has n rows. Past the last chunk e is -1 and seg0, pstart, n describe the last
+// group. Every thread of the block calls it. Up to 256 groups
 // every wave scans the counts by itself, without barriers: a block moves one 128-row tile,
 // and three block-wide scans before it took as long as the tile.
 constexpr int kTailBlocks = 8;  // per slab, for the columns past the last group
@@ -744,7 +744,7 @@ __device__ __forceinline__ GroupChunk find_chunk(const int64_t* __restrict__ cou
     const int ee = t * 4 + i;
     const bool mine = ee < E && ci >= cst[i] && ci < cst[i] + ch[i];
     if (mine || (ci >= total && ee == E - 1)) {
-      g = GroupChunk{mine ? ee : -1, st[i], cst[i] * kTRows, cnt[i], mine ? (ci - cst[i]) * kTRows : ci - total};
+      g = GroupChunk{mine ? ee : -1, st[i], cst[i] * kTRows, cnt[i], mine ? (ci - cst[i]) * kTRows : 0};
       found = true;
     }
   }
@@ -914,21 +914,25 @@ __global__ __launch_bounds__(4 * COLS) void mx_quant_tokens_t_kernel(const uint1
   const int n_chunks = (int)(R / kTRows) + E + kTailBlocks, b = workgroup();
   const int c0 = b / n_chunks * COLS;  // slab-major: blocks running together share column slabs
   if (c0 >= C) return;
-  const GroupChunk gc = find_chunk(counts, R, E, b % n_chunks, s_tmp, &s_gc);
+  // a slab's first blocks are the tail's, which so has its blocks also where the counts sum
+  // up to more than R rows and make more chunks than the launch has blocks (their rows past
+  // R are dropped)
+  const int ci = b % n_chunks - kTailBlocks;
+  const GroupChunk gc = find_chunk(counts, R, E, ci < 0 ? 0x7fffffff : ci, s_tmp, &s_gc);
   const int e = gc.e, seg0 = gc.seg0, pstart = gc.pstart, off = gc.off;
   int n = gc.n;
   if ((int64_t)seg0 + n > R) n = (int)(R - seg0 > 0 ? R - seg0 : 0);
   const int n_out = (n + kMxPad - 1) / kMxPad * kMxPad;
-  if (e < 0) {
+  if (ci < 0) {
     // The columns past the last group, up to Rpad, belong to no group: zero them (and
     // their scale rows) so that every byte of q and s is defined. Both ends are multiples
     // of 32, so the rows' tails take 16-byte stores. Up to E x 127 bytes of each row, by
     // kTailBlocks blocks per slab: one block that also transposed the last group was the
     // launch's last by a sixth of its time (64 groups, 32768 x 2304: 112 -> 93 us).
-    if (off >= kTailBlocks || (int64_t)pstart + n_out > Rpad) return;
+    if ((int64_t)pstart + n_out > Rpad) return;
     constexpr int TC = COLS / kTailBlocks;
     const int64_t end = (int64_t)pstart + n_out, tail16 = (Rpad - end) / 16;
-    const int64_t cb = c0 + off * TC;
+    const int64_t cb = c0 + (ci + kTailBlocks) * TC;
     for (int64_t i = threadIdx.x; i < TC * tail16; i += 4 * COLS) {
       const int64_t c = i / tail16, j = i - c * tail16;
       *(uint4*)(q + (cb + c) * Rpad + end + 16 * j) = make_uint4(0u, 0u, 0u, 0u);
@@ -937,7 +941,7 @@ __global__ __launch_bounds__(4 * COLS) void mx_quant_tokens_t_kernel(const uint1
       s[(end / kMxBlock + i / TC) * C + cb + i % TC] = 0;
     return;
   }
-  if (n <= off || (int64_t)pstart + n_out > Rpad) return;
+  if (e < 0 || n <= off || (int64_t)pstart + n_out > Rpad) return;
   const int64_t r0 = (int64_t)seg0 + off;  // the chunk's first row, and its first token of q
   const int64_t p0 = (int64_t)pstart + off;
   if constexpr (GATHER) {  // this slab's rows and columns of the gathered source
