@@ -173,3 +173,60 @@ def test_token_chunks_more_than_2_32_threads(dev):
     finally:
         del q
         torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("kind", ["fp8_known_amax", "fp8", "mx", "mx_dual", "fp8_more_than_2_32_threads"])
+def test_weight_chunks_in_slices(dev, kind):
+    """Launches of more than one slice of 65536 blocks, and one of 2^23 blocks (1024 experts
+    of 144 x 524288, 154 GB of weights), which is 2^32 threads: every expert repeats 128
+    columns, whose bytes are those of a small launch."""
+    from torchtitan_amd._lib import call, ptr
+
+    huge = kind == "fp8_more_than_2_32_threads"
+    e, a, b = (1024, 144, 1 << 19) if huge else (3, 160, 128 * 21846 if kind == "fp8" else 128 * 10924)
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < e * b * (3 * a + 8) + (8 << 30):
+        pytest.skip(f"needs {e * b * (3 * a + 8) >> 30} GB of free device memory")
+    banner(f"weight quantizer {kind}, {e} x {a} x {b}")
+    gen = torch.Generator(device=dev).manual_seed(9)
+    src = torch.randn(a, 128, generator=gen, device=dev).bfloat16()
+    st = torch.cuda.current_stream().cuda_stream
+
+    def u8(*shape):
+        return torch.full(shape, 0xA5, dtype=torch.uint8, device=dev)
+
+    def quant(e, b):
+        x = torch.empty(e, a, b, dtype=torch.bfloat16, device=dev)
+        x.view(e, a, b // 128, 128).copy_(src[None, :, None, :])
+        if kind.startswith("fp8"):
+            q, s = u8(e, b, a), torch.zeros(e, b, device=dev)
+            if kind == "fp8":
+                call("moe_fp8_quant_cols_t", ptr(x), e, a, b, ptr(q), a * b, a, ptr(s), b, st)
+            else:
+                amax = src.float().abs().amax(0).repeat(e, b // 128)
+                call("moe_fp8_quant_cols_t_amax", ptr(x), ptr(amax), e, a, b, ptr(q), a * b, a, ptr(s), b, st)
+            return [(q, a), (s, 1)]
+        t, ts = u8(e, b, a), u8(e, b, a // 32)
+        args = (ptr(t), a * b, a, ptr(ts), a // 32 * b, a // 32, st)
+        if kind == "mx":
+            call("moe_mxfp8_quant_cols_t", ptr(x), e, a, b, *args)
+            return [(t, a), (ts, a // 32)]
+        q, s = u8(e, a, b), u8(e, a, b // 32)
+        call("moe_mxfp8_quant_dual_cols", ptr(x), e, a, b, ptr(q), ptr(s), *args)
+        return [(t, a), (ts, a // 32), (q, None), (s, None)]
+
+    got = want = None
+    try:
+        want = quant(1, 128)
+        got = quant(e, b)
+        for (t, n), (w, _) in zip(got, want):
+            for i in range(0, e, 73):
+                if n is None:  # row-wise: 128 columns, or their four scales, repeat in each row
+                    assert bool((t[i].view(a, -1, w.shape[2]) == w[0][:, None]).all())
+                else:
+                    assert bool((t[i].view(-1, 128, n) == w.view(128, n)).all()), i
+            if n is not None:  # the last expert's last columns
+                assert bool((t[-1].view(-1, 128, n)[-1] == w.view(128, n)).all())
+    finally:
+        del got, want
+        torch.cuda.empty_cache()

@@ -670,16 +670,17 @@ __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, 
 // known, from quant_rows_colamax_kernel) x is read once, by a block per (e, COLS columns,
 // 128 rows) (ONE); else a block per (e, COLS columns) takes the amax in a pass of its own.
 template <int COLS, bool ONE>
-__global__ __launch_bounds__(4 * COLS) void quant_cols_t_kernel(const uint16_t* __restrict__ x, int A, int B,
+__global__ __launch_bounds__(4 * COLS) void quant_cols_t_kernel(const uint16_t* __restrict__ x, int E, int A, int B,
                                                            uint8_t* __restrict__ q, int64_t q_estride, int64_t q_ld,
                                                            float* __restrict__ scale, int64_t s_estride,
                                                            const float* __restrict__ amax_in) {
   __shared__ float s_red[ONE ? 1 : COLS * 33];
   __shared__ float s_amax[COLS];
   __shared__ __attribute__((aligned(16))) uint32_t s_tile[kTRows * (COLS / 2)];
-  const int nb = B / COLS, nch = ONE ? (A + kTRows - 1) / kTRows : 1;
-  const int64_t e = blockIdx.x / (nb * nch);
-  const int b0 = (blockIdx.x / nch % nb) * COLS, a0 = blockIdx.x % nch * kTRows;
+  const int nb = B / COLS, nch = ONE ? (A + kTRows - 1) / kTRows : 1, w = workgroup();
+  const int64_t e = w / (nb * nch);
+  if (e >= E) return;
+  const int b0 = (w / nch % nb) * COLS, a0 = w % nch * kTRows;
   const uint16_t* base = x + e * A * (int64_t)B + b0;
   if constexpr (ONE) {
     if (threadIdx.x < COLS) s_amax[threadIdx.x] = amax_in[e * B + b0 + threadIdx.x];
@@ -867,14 +868,15 @@ __global__ __launch_bounds__(256) void mx_quant_rows_kernel(const uint4* __restr
 // x [E][A][B] -> q rows (e, b) of A values at q + e * q_estride + b * q_ld, and
 // their A/32 scales at s + e * s_estride + b * s_ld. Block per (e, COLS columns, 128 rows).
 template <int COLS>
-__global__ __launch_bounds__(4 * COLS) void mx_quant_cols_t_kernel(const uint16_t* __restrict__ x, int A, int B,
+__global__ __launch_bounds__(4 * COLS) void mx_quant_cols_t_kernel(const uint16_t* __restrict__ x, int E, int A, int B,
                                                               uint8_t* __restrict__ q, int64_t q_estride,
                                                               int64_t q_ld, uint8_t* __restrict__ s,
                                                               int64_t s_estride, int64_t s_ld) {
   __shared__ __attribute__((aligned(16))) uint32_t s_tile[kTRows * (COLS / 2)];
-  const int nb = B / COLS, nch = (A + kTRows - 1) / kTRows;
-  const int64_t e = blockIdx.x / (nb * nch);
-  const int b0 = (blockIdx.x / nch % nb) * COLS, a0 = blockIdx.x % nch * kTRows, n = min(kTRows, A - a0);
+  const int nb = B / COLS, nch = (A + kTRows - 1) / kTRows, w = workgroup();
+  const int64_t e = w / (nb * nch);
+  if (e >= E) return;
+  const int b0 = (w / nch % nb) * COLS, a0 = w % nch * kTRows, n = min(kTRows, A - a0);
   slab_t_quant<true, false, COLS, false, true, true>(x + (e * A + a0) * (int64_t)B + b0, B, n, n, q + e * q_estride + b0 * q_ld + a0, q_ld,
                             s + e * s_estride + b0 * s_ld + a0 / kMxBlock, s_ld, 1, nullptr, s_tile);
 }
@@ -883,14 +885,15 @@ __global__ __launch_bounds__(4 * COLS) void mx_quant_cols_t_kernel(const uint16_
 // s_r [E][A][B / 32], as mx_quant_rows on [E A, B]) and the transposed one of
 // mx_quant_cols_t. Block per (e, COLS columns, 128 rows).
 template <int COLS>
-__global__ __launch_bounds__(4 * COLS) void mx_dual_cols_kernel(const uint16_t* __restrict__ x, int A, int B,
+__global__ __launch_bounds__(4 * COLS) void mx_dual_cols_kernel(const uint16_t* __restrict__ x, int E, int A, int B,
                                                            uint8_t* __restrict__ q, int64_t q_estride, int64_t q_ld,
                                                            uint8_t* __restrict__ s, int64_t s_estride, int64_t s_ld,
                                                            uint8_t* __restrict__ qr, uint8_t* __restrict__ sr) {
   __shared__ __attribute__((aligned(16))) uint32_t s_tile[kTRows * (COLS / 2)];
-  const int nb = B / COLS, nch = (A + kTRows - 1) / kTRows;
-  const int64_t e = blockIdx.x / (nb * nch);
-  const int b0 = (blockIdx.x / nch % nb) * COLS, a0 = blockIdx.x % nch * kTRows, n = min(kTRows, A - a0);
+  const int nb = B / COLS, nch = (A + kTRows - 1) / kTRows, w = workgroup();
+  const int64_t e = w / (nb * nch);
+  if (e >= E) return;
+  const int b0 = (w / nch % nb) * COLS, a0 = w % nch * kTRows, n = min(kTRows, A - a0);
   const int64_t row0 = e * A + a0;  // the chunk's first row in the [E A, B] view
   slab_t_quant<true, true, COLS, false, true, true>(x + row0 * B + b0, B, n, n, q + e * q_estride + b0 * q_ld + a0, q_ld,
                            s + e * s_estride + b0 * s_ld + a0 / kMxBlock, s_ld, 1, nullptr, s_tile, qr + row0 * B + b0, B,
@@ -1691,10 +1694,10 @@ static int quant_cols_t(const uint16_t* x, const float* col_amax, int32_t n_expe
   const auto k128 = one ? quant_cols_t_kernel<128, true> : quant_cols_t_kernel<128, false>;
   const auto k64 = one ? quant_cols_t_kernel<64, true> : quant_cols_t_kernel<64, false>;
   if (b % 128 == 0)
-    hipLaunchKernelGGL(k128, dim3(n_experts * (b / 128) * n_chunks), dim3(512), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(k128, sliced((int64_t)n_experts * (b / 128) * n_chunks), dim3(512), 0, stream, x, n_experts, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, col_amax);
   else
-    hipLaunchKernelGGL(k64, dim3(n_experts * (b / 64) * n_chunks), dim3(256), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(k64, sliced((int64_t)n_experts * (b / 64) * n_chunks), dim3(256), 0, stream, x, n_experts, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, col_amax);
   return launch_status();
 }
@@ -1988,10 +1991,10 @@ MOE_API int moe_mxfp8_quant_cols_t(const uint16_t* x, int32_t n_experts, int32_t
   if (!x || !q || !scale) return kErrInvalidArgument;
   const int n_chunks = (a + kTRows - 1) / kTRows;
   if (b % 128 == 0)
-    hipLaunchKernelGGL(mx_quant_cols_t_kernel<128>, dim3(n_experts * (b / 128) * n_chunks), dim3(512), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(mx_quant_cols_t_kernel<128>, sliced((int64_t)n_experts * (b / 128) * n_chunks), dim3(512), 0, stream, x, n_experts, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, scale_row_stride);
   else
-    hipLaunchKernelGGL(mx_quant_cols_t_kernel<64>, dim3(n_experts * (b / 64) * n_chunks), dim3(256), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(mx_quant_cols_t_kernel<64>, sliced((int64_t)n_experts * (b / 64) * n_chunks), dim3(256), 0, stream, x, n_experts, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, scale_row_stride);
   return launch_status();
 }
@@ -2030,10 +2033,10 @@ MOE_API int moe_mxfp8_quant_dual_cols(const uint16_t* x, int32_t n_experts, int3
   if (!x || !q || !scale || !q_rows || !scale_rows) return kErrInvalidArgument;
   const int n_chunks = (a + kTRows - 1) / kTRows;
   if (b % 128 == 0)
-    hipLaunchKernelGGL(mx_dual_cols_kernel<128>, dim3(n_experts * (b / 128) * n_chunks), dim3(512), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(mx_dual_cols_kernel<128>, sliced((int64_t)n_experts * (b / 128) * n_chunks), dim3(512), 0, stream, x, n_experts, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, scale_row_stride, q_rows, scale_rows);
   else
-    hipLaunchKernelGGL(mx_dual_cols_kernel<64>, dim3(n_experts * (b / 64) * n_chunks), dim3(256), 0, stream, x, a, b, q,
+    hipLaunchKernelGGL(mx_dual_cols_kernel<64>, sliced((int64_t)n_experts * (b / 64) * n_chunks), dim3(256), 0, stream, x, n_experts, a, b, q,
                        q_expert_stride, q_row_stride, scale, scale_expert_stride, scale_row_stride, q_rows, scale_rows);
   return launch_status();
 }
