@@ -83,6 +83,15 @@ def test_cases_take_their_tiles(oss):
     assert taken == tiles_of(oss)
 
 
+@pytest.mark.parametrize("oss", [False, True], ids=["swiglu", "gptoss"])
+@pytest.mark.parametrize("e,d,h", [(256, 2304, 1024), (64, 2048, 1408), (32, 7168, 2048), (128, 2880, 2880)])
+def test_experts_without_a_row_do_not_change_the_tile(oss, e, d, h):
+    """With no more rows than experts the row kernels take the tile of that many experts."""
+    for rows in range(1, e):
+        for m in MODES[:4]:
+            assert tile(m, oss, e, d, h, rows) == tile(m, oss, rows, d, h, rows), (m, rows)
+
+
 def _close(a, b, what, tol):
     den = b.abs().max().item()
     err = (a.float() - b).abs().max().item() / (den if den > 0 else 1.0)
