@@ -92,6 +92,15 @@ def test_experts_without_a_row_do_not_change_the_tile(oss, e, d, h):
             assert tile(m, oss, e, d, h, rows) == tile(m, oss, rows, d, h, rows), (m, rows)
 
 
+@pytest.mark.parametrize("e,d,h,rows", [(64, 3072, 1536, 6701), (256, 2304, 1024, 23480), (128, 1536, 768, 30816),
+                                        (64, 2304, 1024, 600), (24, 1536, 320, 44073)])
+def test_dx_on_whole_384_tiles(e, d, h, rows):
+    """Where D is a multiple of 384 and rounds do not speak clearly for another tile, dx stays on
+    128 x 384, measured 5 to 30 % faster at these shapes than the tiles that cost a little less
+    by their rounds."""
+    assert tile("dx", False, e, d, h, rows) == DX384
+
+
 def _close(a, b, what, tol):
     den = b.abs().max().item()
     err = (a.float() - b).abs().max().item() / (den if den > 0 else 1.0)

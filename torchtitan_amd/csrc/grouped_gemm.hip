@@ -959,8 +959,12 @@ static void launch_cfg(const GemmParams& p, int64_t R, hipStream_t stream) {
 //                  an expert has more than one tile of rows (with fewer the weights'
 //                  bytes bound every tile)
 //  dx              128 x 256, 32-wide, 3 stages                1.0
-//                  128 x 384                                   1.45; 1.55 where no expert
-//                  has more than one tile of rows (the narrow tile streams weights faster)
+//                  128 x 384                                   1.45, 1.15 where D is a
+//                  multiple of 384 (no partial tiles; with 1.45 there too, 40 of 259 measured
+//                  shapes were over 3 % slower than on this tile, by up to a third, now 7: us,
+//                  3072 / 1536 / 64 / 6701 345 -> 271, 2304 / 1024 / 256 / 23480 538 -> 503,
+//                  1536 / 768 / 128 / 30816 266 -> 231); 1.07 times that where no expert has
+//                  more than one tile of rows (the narrow tile streams weights faster)
 //                  128 x 512                                   1.73, where D is a multiple of
 //                  512 (its w1 half is parked in the dx rows: a partial tile wastes that
 //                  traffic too); the gpt-oss dx parks nothing and takes it at any D, and
@@ -1008,7 +1012,7 @@ static GemmTile pick_tile(int mode, int act, int64_t R, int64_t E, int64_t D, in
   }
   if (mode == kBwdDx) {
     const double c256 = rounds(m128 * n_tiles(D, 256), cus),
-                 c384 = (m128 > least ? 1.45 : 1.55) * rounds(m128 * n_tiles(D, 384), cus),
+                 c384 = (D % 384 ? 1.45 : 1.15) * (m128 > least ? 1.0 : 1.07) * rounds(m128 * n_tiles(D, 384), cus),
                  c512 = act == kOssGLU || D % 512 == 0 ? 1.73 * rounds(m128 * n_tiles(D, 512), cus) : INFINITY,
                  c_two = 1.95 * rounds(m128 * n_tiles(D, 256), 2 * cus),
                  c_tall = act == kOssGLU ? 1.62 * rounds(m256 * n_tiles(D, 256), cus) : INFINITY;
