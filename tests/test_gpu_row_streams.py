@@ -50,3 +50,40 @@ def test_rows_equal_torch(dev, n, d, e, k, dtype, scored):
         for got, other in ((got_s, x[token_idx]), (got_cs, go[token_idx])):
             p = rows.double() * other.double()
             assert ((got.double() - p.sum(1)).abs() <= d * 2.0 ** -24 * p.abs().sum(1)).all()
+
+
+def test_small_combine_keeps_its_rows(dev):
+    """Below the streaming size the combine leaves its rows in the caches, where a scored
+    backward that follows at once (a recomputed layer) finds them: it takes about as long as
+    when its rows were just read by the backward itself. With rows read past the caches it
+    took 1.5 times as long at this size (59 MB of rows)."""
+    from torchtitan_amd import ops
+
+    n, d, e, k = 512, 7168, 64, 8
+    banner("combine of 59 MB of rows, then its scored backward")
+    gen = torch.Generator(device=dev).manual_seed(3)
+    idx = torch.rand(n, e, device=dev, generator=gen).topk(k).indices
+    scores, _idx, _counts, _offs, slot_pos, tok_pos = ops.reorder(torch.rand(n, k, device=dev, generator=gen), idx, e)
+    shared, go = (torch.randn(n, d, device=dev, generator=gen).bfloat16() for _ in range(2))
+    rows = torch.randn(n * k, d, device=dev, generator=gen).bfloat16()
+    flush = torch.empty(1 << 28, dtype=torch.int32, device=dev)
+
+    def backward():
+        ops.combine_backward(go, rows, slot_pos, tok_pos, scores)
+
+    def timed(first):
+        times = []
+        for _ in range(9):
+            flush.zero_()  # 1 GB: nothing of the rows is left in the caches
+            first()
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            backward()
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return sorted(times)[4]
+
+    timed(backward)
+    own, after = timed(backward), timed(lambda: ops.combine(shared, rows, slot_pos, tok_pos, scores))
+    assert after < 1.25 * own, (after, own)

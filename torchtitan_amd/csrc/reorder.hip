@@ -309,10 +309,12 @@ __global__ __launch_bounds__(256) void expand_rows_kernel(const T* __restrict__ 
 // sorted index_put with accumulate); r_k = routed[pos_k], or
 // round(routed[pos_k] * score) when the score is applied after the experts
 // (moe.py:465-469). Without a shared expert the sum starts from zero.
-// Bound by reading the routed rows, once each: their loads do not keep them in the caches
-// (timed after the kernel that writes them: 154 -> 134 us for 604 MB of
+// Bound by reading the routed rows, once each. STREAM (past kStreamBytes): their loads do not
+// keep them in the caches (timed after the kernel that writes them: 154 -> 134 us for 604 MB of
 // bf16 rows, 132 -> 105 for 537 MB of fp32, 74 -> 64 for 302 MB, 18 for 75 MB either way).
-template <typename T, int MAXK>
+// Below the line they are kept for the scored backward, which reads them again at once where
+// a layer is recomputed (512 tokens of 7168, K = 8: that backward 80 us with rows that are not, 52 with rows that are).
+template <typename T, int MAXK, bool STREAM>
 __global__ __launch_bounds__(256) void combine_kernel(const T* __restrict__ shared_out,
                                                       const T* __restrict__ routed,
                                                       const int32_t* __restrict__ tok_pos,
@@ -339,8 +341,10 @@ __global__ __launch_bounds__(256) void combine_kernel(const T* __restrict__ shar
     }
     uint4 v[MAXK];
 #pragma unroll
-    for (int k = 0; k < MAXK; ++k)
-      v[k] = k < K ? nt_load(routed + (int64_t)pos[k] * D + ch * n) : make_uint4(0, 0, 0, 0);
+    for (int k = 0; k < MAXK; ++k) {
+      const T* row = routed + (int64_t)pos[k] * D + ch * n;
+      v[k] = k >= K ? make_uint4(0, 0, 0, 0) : (STREAM ? nt_load(row) : *(const uint4*)row);
+    }
 #pragma unroll
     for (int k = 0; k < MAXK; ++k) {
       if (k < K) {
@@ -631,16 +635,12 @@ static void launch_expand(const void* src, int64_t n_tokens, int dim, int top_k,
 template <typename T>
 static void launch_combine(const void* shared_out, const void* routed, const int32_t* tok_pos, const float* scores,
                            int64_t n_tokens, int dim, int top_k, void* out, hipStream_t stream) {
-  const dim3 grid(stream_grid(n_tokens * (dim / Chunk<T>::kN), 256, 32768));
-  if (top_k <= 8)
-    hipLaunchKernelGGL((combine_kernel<T, 8>), grid, dim3(256), 0, stream, (const T*)shared_out, (const T*)routed,
-                       tok_pos, scores, n_tokens, dim, top_k, (T*)out);
-  else if (top_k <= 16)
-    hipLaunchKernelGGL((combine_kernel<T, 16>), grid, dim3(256), 0, stream, (const T*)shared_out, (const T*)routed,
-                       tok_pos, scores, n_tokens, dim, top_k, (T*)out);
-  else
-    hipLaunchKernelGGL((combine_kernel<T, kMaxTopK>), grid, dim3(256), 0, stream, (const T*)shared_out,
-                       (const T*)routed, tok_pos, scores, n_tokens, dim, top_k, (T*)out);
+  const bool nt = streamed<T>(n_tokens, dim, top_k);
+  auto* kernel = top_k <= 8    ? (nt ? combine_kernel<T, 8, true> : combine_kernel<T, 8, false>)
+                 : top_k <= 16 ? (nt ? combine_kernel<T, 16, true> : combine_kernel<T, 16, false>)
+                               : (nt ? combine_kernel<T, kMaxTopK, true> : combine_kernel<T, kMaxTopK, false>);
+  hipLaunchKernelGGL(kernel, dim3(stream_grid(n_tokens * (dim / Chunk<T>::kN), 256, 32768)), dim3(256), 0, stream,
+                     (const T*)shared_out, (const T*)routed, tok_pos, scores, n_tokens, dim, top_k, (T*)out);
 }
 
 template <typename T, int MAXK, bool STREAM>
