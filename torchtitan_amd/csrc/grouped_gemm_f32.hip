@@ -141,21 +141,24 @@ __device__ __forceinline__ void find_tile(const Params& p, int ntn, int* s_tmp, 
   mt = bx - s_out[3];
 }
 
-// dW: start and count of expert e's rows
-__device__ __forceinline__ void find_segment(const int64_t* counts, int64_t R, int E, int e, int* s_tmp, int* s_out,
-                                             Seg& seg) {
-  int cnt[4], st[4];
-  scan_counts(counts, R, E, s_tmp, st, cnt);
+// dW: start and count of expert e's rows, cut where they run past R. Every wave adds up the
+// counts before e by itself (each sum cut at R: none wraps), without barriers: where an expert
+// has few rows a workgroup is little more than this, two copies and its stores.
+__device__ __forceinline__ Seg find_segment(const int64_t* counts, int64_t R, int e, int lane) {
+  const uint32_t most = (uint32_t)R;
+  auto cut = [&](int64_t c) { return c < 0 ? 0u : (c > R ? most : (uint32_t)c); };
+  uint32_t start = 0;
+  for (int base = 0; base < e; base += 256) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if ((int)threadIdx.x * 4 + i == e) {
-      s_out[0] = st[i];
-      s_out[1] = cnt[i];
+    for (int i = 0; i < 4; ++i) {
+      const int ee = base + 4 * lane + i;
+      if (ee < e) start = min(start + cut(counts[ee]), most);
     }
   }
-  __syncthreads();
-  seg.start = s_out[0];
-  seg.count = s_out[1];
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) start = min(start + (uint32_t)__shfl_xor((int)start, off), most);
+  start = __builtin_amdgcn_readfirstlane(start);
+  return Seg{(int)start, (int)min(cut(counts[e]), most - start)};
 }
 
 // A wave copies two of an operand's eight 1 KB pieces (8 rows, or 4 k-rows) of a stage.
@@ -304,6 +307,10 @@ __global__ __launch_bounds__(512, MODE == kGateUp ? 6 : 8) void rows_kernel(Para
 // Weight gradients: out[e][m][n] = sum over expert e's rows r of a[r][m] b[r][n], up to
 // three products per launch (each alone has too few tiles to fill the chip at the sizes
 // this path is used at). Waves: 32 x 32 each.
+// NS stages. One where experts have few rows (launch_dw): such a workgroup waits for its one
+// stage and writes its tile, and with half the LDS eight of them share a CU instead of five;
+// its last stage is copied and multiplied only up to 16 rows where it has no more (the test
+// costs the long loop of two stages 2 to 5 %).
 struct DwJob {
   const float* a;  // [R, M]
   const float* b;  // [R, N]
@@ -319,12 +326,10 @@ struct DwParams {
   DwJob job[3];
 };
 
-template <bool ALIGNED>
+template <bool ALIGNED, int NS>
 __global__ __launch_bounds__(256, 4) void dw_kernel(DwParams p) {
-  __shared__ __attribute__((aligned(1024))) float sA[2][kTile];
-  __shared__ __attribute__((aligned(1024))) float sB[2][kTile];
-  __shared__ int s_tmp[8];
-  __shared__ int s_out[2];
+  __shared__ __attribute__((aligned(1024))) float sA[NS][kTile];
+  __shared__ __attribute__((aligned(1024))) float sB[NS][kTile];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // Workgroup b runs on XCD b % 8. Every XCD takes an eighth of each (job, expert)'s tiles,
   // neighbouring ones: whole experts per XCD would share more in its L2 but leave XCDs
@@ -339,12 +344,12 @@ __global__ __launch_bounds__(256, 4) void dw_kernel(DwParams p) {
   const DwJob job = ji == 0 ? p.job[0] : (ji == 1 ? p.job[1] : p.job[2]);
   const int M = job.M, N = job.N, ntn = N / BN;
   const int m0 = (t / ntn) * BM, n0 = (t % ntn) * BN;
-  Seg seg;
-  find_segment(p.counts, p.R, p.E, e, s_tmp, s_out, seg);
+  const Seg seg = find_segment(p.counts, p.R, e, lane);
   const int wm = w >> 1, wn = w & 1, g = lane >> 4, li = lane & 15;
   const float* A = job.a + (int64_t)seg.start * M + m0;
   const float* B = job.b + (int64_t)seg.start * N + n0;
   auto issue = [&](int k0, int s) {
+    if (NS == 1 && w >= 2 && k0 + BK / 2 >= seg.count) return;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int cc = 2 * w + c, k = k0 + krow_of(cc, lane), col = krow_chunk(cc, lane) * 4;
@@ -359,11 +364,12 @@ __global__ __launch_bounds__(256, 4) void dw_kernel(DwParams p) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   if (seg.count > 0) issue(0, 0);
-  for (int k0 = 0, s = 0; k0 < seg.count; k0 += BK, s ^= 1) {
+  for (int k0 = 0, s = 0; k0 < seg.count; k0 += BK, s ^= NS - 1) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (k0 + BK < seg.count) issue(k0 + BK, s ^ 1);
+    if (NS == 2 && k0 + BK < seg.count) issue(k0 + BK, s ^ 1);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      if (NS == 1 && h == 1 && k0 + BK / 2 >= seg.count) break;
       f32x2_t av[4], bv[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -378,13 +384,28 @@ __global__ __launch_bounds__(256, 4) void dw_kernel(DwParams p) {
           for (int i = 0; i < 2; ++i)
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[s4][j], av[s4][i], acc[i][j], 0, 0, 0);
     }
+    if (NS == 1 && k0 + BK < seg.count) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave has read the stage
+      issue(k0 + BK, 0);
+    }
   }
-  // m-tile i holds rows 32 wm + 2 li + i; a lane's columns are 32 wn + 8 g .. + 7
+  // m-tile i holds rows 32 wm + 2 li + i; a lane's columns are 32 wn + 8 g .. + 7, two 16-byte
+  // pieces. The lanes of a row exchange them so that each store writes 64 whole bytes of 16 rows
+  // (lane group g pieces g and 4 + g).
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    float* o = job.out + ((int64_t)e * M + m0 + 32 * wm + 2 * li + i) * N + n0 + 32 * wn + 8 * g;
-    *(f32x4_u*)o = f32x4_t{acc[i][0][0], acc[i][1][0], acc[i][0][1], acc[i][1][1]};
-    *(f32x4_u*)(o + 4) = f32x4_t{acc[i][0][2], acc[i][1][2], acc[i][0][3], acc[i][1][3]};
+    float* o = job.out + ((int64_t)e * M + m0 + 32 * wm + 2 * li + i) * N + n0 + 32 * wn + 4 * g;
+    f32x4_t lo, hi;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[i][v & 1][v >> 1]),
+                                                      __float_as_uint(acc[i][v & 1][2 + (v >> 1)]), false, false);
+      const auto y = __builtin_amdgcn_permlane32_swap(x[0], x[1], false, false);
+      lo[v] = __uint_as_float(y[0]);
+      hi[v] = __uint_as_float(y[1]);
+    }
+    *(f32x4_u*)o = lo;
+    *(f32x4_u*)(o + 16) = hi;
   }
 }
 
@@ -459,8 +480,15 @@ int launch_dw(DwParams& p, int jobs, hipStream_t stream) {
   p.tiles = (int)grid;
   bool aligned = true;
   for (int j = 0; j < jobs; ++j) aligned = aligned && aligned16(p.job[j].a, p.job[j].b, nullptr, nullptr);
-  if (aligned) hipLaunchKernelGGL(dw_kernel<true>, sliced(grid), dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL(dw_kernel<false>, sliced(grid), dim3(256), 0, stream, p);
+  // up to 64 rows per expert, two stages or fewer. All three weights, us, against three launches
+  // of 16-row stages, with two stages | with one: 64 experts of 1024 / 704, backward of 250 rows
+  // 348 -> 369 | 330, of 1000 with 300 in use 340 -> 376 | 334, 1000 in use 412 -> 387 | 352;
+  // past the line two stages win where the chip is not full: 8 experts of 256 / 512, 1000 rows
+  // 57 | 59, 8000 rows 195 | 209
+  const bool few = p.R <= 64 * (int64_t)p.E;
+  auto* kernel = aligned ? (few ? dw_kernel<true, 1> : dw_kernel<true, 2>)
+                         : (few ? dw_kernel<false, 1> : dw_kernel<false, 2>);
+  hipLaunchKernelGGL(kernel, sliced(grid), dim3(256), 0, stream, p);
   return launch_status();
 }
 
