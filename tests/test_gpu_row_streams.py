@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 # (tokens, dim, experts, top_k, dtype): up to 187 MB of sorted rows
 CASES = [(37, 8, 8, 1, torch.bfloat16), (100, 520, 16, 8, torch.bfloat16), (61, 264, 32, 9, torch.float32),
          (300, 1000, 32, 17, torch.bfloat16), (5600, 2048, 64, 8, torch.bfloat16), (5700, 2048, 64, 8, torch.bfloat16),
-         (5640, 1024, 16, 8, torch.float32), (5600, 1024, 16, 8, torch.float32)]
+         (5640, 1024, 16, 8, torch.float32), (5600, 1024, 16, 8, torch.float32),
+         (50, 264, 32, 12, torch.bfloat16), (3072, 72, 32, 16, torch.bfloat16), (3073, 72, 32, 16, torch.bfloat16)]
 
 
 @pytest.mark.parametrize("scored", [True, False], ids=["scored", "plain"])

@@ -372,16 +372,17 @@ __device__ __forceinline__ int token_wave() {
 
 // Backward of the combine when the score is applied after the experts:
 //   grad_routed[pos] = round(grad_out[t] * s[pos]);  grad_s[pos] = sum_d grad_out[t,d] * routed[pos,d]
-// One wavefront per token, its positions scalar for K in 9..16 (4096 tokens of 2304, K = 16:
-// 178 -> 141 us); with fewer they fit the vector registers and scalar ones win 7 % at 1024
-// columns but lose 3 to 5 % from 2304 on.
-template <typename T, int MAXK>
+// One wavefront per token. SCALAR: its positions as scalars, for K in 9..16 in bf16 where the
+// tokens are more than one round of the other form (launch_combine_bwd_scored); with fewer
+// experts they fit the vector registers and scalar ones win 7 % at 1024 columns but lose 3 to
+// 5 % from 2304 on.
+template <typename T, int MAXK, bool SCALAR>
 __global__ __launch_bounds__(256) void combine_bwd_scored_kernel(
     const T* __restrict__ grad_out, const T* __restrict__ routed, const int32_t* __restrict__ tok_pos,
     const float* __restrict__ scores_sorted, int64_t n_tokens, int D, int K, T* __restrict__ grad_routed,
     float* __restrict__ grad_scores) {
   constexpr int n = Chunk<T>::kN;
-  const int lane = threadIdx.x & 63, wv = sizeof(T) == 2 && MAXK == 16 ? token_wave<MAXK>() : threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = SCALAR ? token_wave<MAXK>() : threadIdx.x >> 6;
   const int cpr = D / n;
   for (int64_t t = (int64_t)blockIdx.x * 4 + wv; t < n_tokens; t += (int64_t)gridDim.x * 4) {
     float part[MAXK];
@@ -673,16 +674,19 @@ template <typename T>
 static void launch_combine_bwd_scored(const void* grad_out, const void* routed, const int32_t* tok_pos,
                                       const float* scores, int64_t n_tokens, int dim, int top_k,
                                       void* grad_routed, float* grad_scores, hipStream_t stream) {
-  const dim3 grid(stream_grid(n_tokens, 4, 16384));
-  if (top_k <= 8)
-    hipLaunchKernelGGL((combine_bwd_scored_kernel<T, 8>), grid, dim3(256), 0, stream, (const T*)grad_out,
-                       (const T*)routed, tok_pos, scores, n_tokens, dim, top_k, (T*)grad_routed, grad_scores);
-  else if (top_k <= 16)
-    hipLaunchKernelGGL((combine_bwd_scored_kernel<T, 16>), grid, dim3(256), 0, stream, (const T*)grad_out,
-                       (const T*)routed, tok_pos, scores, n_tokens, dim, top_k, (T*)grad_routed, grad_scores);
-  else
-    hipLaunchKernelGGL((combine_bwd_scored_kernel<T, kMaxTopK>), grid, dim3(256), 0, stream, (const T*)grad_out,
-                       (const T*)routed, tok_pos, scores, n_tokens, dim, top_k, (T*)grad_routed, grad_scores);
+  // The kernel for 9 to 16 experts runs three waves a SIMD with its positions in vector registers
+  // (160 of them): 3072 tokens a round. Up to there that is the faster form, past it the one with
+  // scalar positions, seven waves but a chain of scalar loads before the rows (us, vector |
+  // scalar: K = 12, 2000 tokens of 256 15.6 | 18.4, 3000 of 2304 74 | 77, 4096 of 2304 127 | 92,
+  // 16384 of 256 79 | 60, 8192 of 7168 622 | 616).
+  constexpr bool kScalar = sizeof(T) == 2;
+  const bool scalar = kScalar && n_tokens > 3072;
+  auto* kernel = top_k <= 8    ? combine_bwd_scored_kernel<T, 8, false>
+                 : top_k <= 16 ? (scalar ? combine_bwd_scored_kernel<T, 16, kScalar>
+                                         : combine_bwd_scored_kernel<T, 16, false>)
+                               : combine_bwd_scored_kernel<T, kMaxTopK, false>;
+  hipLaunchKernelGGL(kernel, dim3(stream_grid(n_tokens, 4, 16384)), dim3(256), 0, stream, (const T*)grad_out,
+                     (const T*)routed, tok_pos, scores, n_tokens, dim, top_k, (T*)grad_routed, grad_scores);
 }
 
 MOE_API int moe_permute(const void* x, const int32_t* slot_pos, const float* scores_sorted,
