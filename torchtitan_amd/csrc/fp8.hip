@@ -461,14 +461,14 @@ constexpr int kTRows = 128;  // slab rows transposed per pass
 //  * ROWS (MX): the same read also quantizes the slab along its columns (the
 //    row-wise MX layout, blocks of 32 columns): row r's COLS values go to
 //    qr + r * ldr and its COLS / 32 block scales to sr + r * ldsr.
-// A pass moves 128 rows (four 16-byte loads per thread, double-buffered in
-// registers so that two passes' loads are in flight) through s_tile
+// A pass moves 128 rows (four 16-byte loads per thread) through s_tile
 // (128 row-major rows of 2 COLS bytes, written with 16-byte stores, the 16-byte
 // chunk c of row r at c ^ ((r / 16) % 8)). Each thread then quantizes two units
 // of 16 rows of one column (2-byte reads; the swizzle keeps the eight row
 // groups a wave reads at once in distinct banks) and stores their 16 bytes, so
-// that 8 consecutive lanes write 128 contiguous bytes of one output row. The
-// loads two passes ahead are issued as soon as the tile is in LDS.
+// that 8 consecutive lanes write 128 contiguous bytes of one output row.
+// Not ONE (fp8 without GATHER): the passes are double-buffered in registers, the loads
+// two passes ahead issued as soon as a tile is in LDS.
 // ONE: the slab is a single pass of at most 128 rows. Nothing is loaded ahead, so a
 // thread needs half the registers (107-116 -> 55 VGPRs) and four blocks share a CU
 // instead of two, and a launch has blocks for every 128 rows: the other blocks, and not
@@ -482,14 +482,14 @@ constexpr int kTRows = 128;  // slab rows transposed per pass
 // the passes. 128-column
 // slabs (launched whenever the width allows) write the row-wise layout in whole
 // 128-byte lines: 2-12 % faster than 64-column ones at the Kimi shapes.
-// GATHER: the slab's rows are gathered (RowGather); the indices are loaded two
-// passes ahead of the rows they address and the scale is applied when a pass is
-// consumed, so neither waits behind the row loads in flight.
-// NT: weights, read past the caches (this is their last reader in a pass). Experts'
-// forward / backward in us, kept / not kept: MX forward 48 x 768 x 1280 234 -> 220, fp8
-// backward 352 -> 338, 16 x 1536 x 4096 967 -> 940, 64 x 1024 x 2304 825 -> 799 (4096 rows);
-// MX forward of the other two 560 -> 567 and 557 -> 556. Token rows are read again by the
-// next kernel and gain nothing (fp8 backward of 1024 rows 1 % slower).
+// GATHER: the slab's rows are gathered (RowGather); the scale is applied when the
+// pass is consumed.
+// NT: weights, read past the caches (this is their last reader in a pass). us, kept / not
+// kept: MX dual cols 64 x 2304 x 1024 (the first of a pass) 145 -> 120, the others 123 -> 121;
+// 48 x 768 x 1280 48 -> 43; 16 x 4096 x 1536 100 -> 81; fp8 cols 64 x 1024 x 2304 84 -> 79, 16 x
+// 4096 x 1536 59 -> 53. Experts' forward and backward of 64 to 32768 rows 0 to 5 % faster, none
+// slower by more than its runs differ. Token rows are read again by the next kernel and gain
+// nothing (fp8 backward of 1024 rows 1 % slower).
 template <bool MX, bool ROWS, int COLS, bool GATHER = false, bool ONE = false, bool NT = false>
 __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, int64_t ld, int n_rows, int n_out,
                                              uint8_t* __restrict__ out, int64_t ldo, uint8_t* __restrict__ sc,
@@ -497,9 +497,10 @@ __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, 
                                              uint8_t* __restrict__ qr = nullptr, int64_t ldr = 0,
                                              uint8_t* __restrict__ sr = nullptr, int64_t ldsr = 0,
                                              RowGather gather = RowGather{}) {
+  static_assert(ONE || !(MX || GATHER), "only the fp8 quantizers that take their own amax run several passes");
   constexpr int T = 4 * COLS, CPR = COLS / 8;
   const int t = threadIdx.x;
-  auto in_rows = [&](int row) { return row >= 0 && row < n_rows; };
+  auto in_rows = [&](int row) { return row < n_rows; };
   // Barriers wait for LDS only: __syncthreads() would also drain the global loads
   // of the passes ahead and the stores behind (its workgroup-scope fence is a
   // vmcnt(0)), which left one pass in flight. The tile's NaN flag is one word
@@ -507,23 +508,21 @@ __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, 
   // next pass's writes come after its first barrier, so one set of words does).
   __shared__ uint32_t s_wnan[T / 64];
   auto lds_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-  uint4 va[4], vb[4];
-  int64_t ia[4], ib[4];  // GATHER: source rows of the pass two ahead of va / vb
-  float sa[4], sb[4];    // GATHER with scale: the row scales of the pass in va / vb
+  int64_t ix[4];    // GATHER: the rows' source rows
+  float sv[4];      // GATHER with scale: their scales
+  uint32_t ok = 0;  // GATHER: bit i where load i reads a row of the slab with a source row in range
   // Every load is issued, rows outside the slab (and passes past its end) reading
   // a clamped row whose value is then dropped: with no load skipped on any path,
   // the compiler counts the loads in flight and waits for one pass's rows with
   // vmcnt(N) rather than vmcnt(0), which drained the pass ahead as well.
   // The rows' values are zeroed where they are consumed (zero_rows), not where they
   // are loaded: a select right after a load makes the load's wait immediate.
-  auto clamp_row = [&](int row) { return row < 0 ? 0 : (row >= n_rows ? n_rows - 1 : row); };
-  auto load_idx = [&](int64_t (&ix)[4], int a0) {
+  auto clamp_row = [&](int row) { return row >= n_rows ? n_rows - 1 : row; };
+  auto load = [&](uint4 (&v)[4], int a0) {
+    if constexpr (GATHER) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ix[i] = gather.idx[clamp_row(a0 + (t + i * T) / CPR)];
-  };
-  // GATHER: ok gets bit i when load i reads a row of the slab with a source row in range
-  auto load = [&](uint4 (&v)[4], const int64_t (&ix)[4], float (&sv)[4], uint32_t& ok, int a0) {
-    ok = 0;
+      for (int i = 0; i < 4; ++i) ix[i] = gather.idx[clamp_row(a0 + (t + i * T) / CPR)];
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int c = t + i * T;
@@ -540,14 +539,14 @@ __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, 
       }
     }
   };
-  auto zero_rows = [&](uint4 (&v)[4], uint32_t ok, int a0) {
+  auto zero_rows = [&](uint4 (&v)[4], int a0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const bool in = GATHER ? ((ok >> i) & 1u) != 0u : in_rows(a0 + (t + i * T) / CPR);
       if (!in) v[i] = make_uint4(0, 0, 0, 0);
     }
   };
-  auto apply_scales = [&](uint4 (&v)[4], const float (&sv)[4], int a0) {
+  auto apply_scales = [&](uint4 (&v)[4], int a0) {
     if constexpr (GATHER) {
       if (!gather.scale) return;
 #pragma unroll
@@ -557,11 +556,11 @@ __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, 
       }
     }
   };
-  // one pass of 128 rows held in v; v is reloaded with the pass two ahead as soon
-  // as it is in LDS, so two passes' loads are in flight while one is transposed
-  auto pass = [&](uint4 (&v)[4], int64_t (&ix)[4], float (&sv)[4], uint32_t& ok, int a0) {
-    zero_rows(v, ok, a0);
-    apply_scales(v, sv, a0);
+  // one pass of 128 rows held in v; if not ONE, v is reloaded with the pass two ahead as
+  // soon as it is in LDS, so two passes' loads are in flight while one is transposed
+  auto pass = [&](uint4 (&v)[4], int a0) {
+    zero_rows(v, a0);
+    apply_scales(v, a0);
     const uint32_t nan = has_nan8(v[0]) | has_nan8(v[1]) | has_nan8(v[2]) | has_nan8(v[3]);
     if constexpr (ROWS) {
       const bool rows_fast = wave_nan_free(nan);
@@ -596,10 +595,7 @@ __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, 
 #pragma unroll
     for (int w = 0; w < T / 64; ++w) any_nan |= s_wnan[w];
     const bool fast = any_nan == 0u;  // block-uniform: the tile holds no NaN
-    if constexpr (!ONE) {
-      load(v, ix, sv, ok, a0 + 2 * kTRows);
-      if constexpr (GATHER) load_idx(ix, a0 + 4 * kTRows);
-    }
+    if constexpr (!ONE) load(v, a0 + 2 * kTRows);
     // unit (column cc, rows 16 kq .. 16 kq + 15 of the pass): 8 consecutive lanes cover one
     // output row's 128 bytes, so every store instruction writes 8 rows x 128 contiguous bytes
 #pragma unroll
@@ -637,31 +633,24 @@ __device__ __forceinline__ void slab_t_quant(const uint16_t* __restrict__ base, 
           for (int bq = 0; bq < 4; ++bq) o[q] |= e4m3(xv[4 * q + bq] * f) << (8 * bq);
         }
       }
-      if (rb >= 0 && rb < n_out) {
+      if (rb < n_out) {
         *(uint4*)(out + (int64_t)cc * ldo + rb) = make_uint4(o[0], o[1], o[2], o[3]);
         if constexpr (MX)
           if ((kq & 1) == 0) sc[(int64_t)cc * sc_b + (int64_t)(rb / kMxBlock) * sc_k] = (uint8_t)e;
       }
     }
   };
-  uint32_t oka, okb;
+  uint4 va[4];
+  load(va, 0);
   if constexpr (ONE) {
-    if constexpr (GATHER) load_idx(ia, 0);
-    load(va, ia, sa, oka, 0);
-    pass(va, ia, sa, oka, 0);
-    return;
-  }
-  if constexpr (GATHER) {
-    load_idx(ia, 0);
-    load_idx(ib, kTRows);
-  }
-  load(va, ia, sa, oka, 0);
-  if constexpr (GATHER) load_idx(ia, 2 * kTRows);
-  load(vb, ib, sb, okb, kTRows);
-  if constexpr (GATHER) load_idx(ib, 3 * kTRows);
-  for (int a0 = 0; a0 < n_out; a0 += 2 * kTRows) {
-    pass(va, ia, sa, oka, a0);
-    if (a0 + kTRows < n_out) pass(vb, ib, sb, okb, a0 + kTRows);
+    pass(va, 0);
+  } else {
+    uint4 vb[4];
+    load(vb, kTRows);
+    for (int a0 = 0; a0 < n_out; a0 += 2 * kTRows) {
+      pass(va, a0);
+      if (a0 + kTRows < n_out) pass(vb, a0 + kTRows);
+    }
   }
 }
 
@@ -775,7 +764,6 @@ __global__ __launch_bounds__(4 * COLS) void quant_tokens_t_kernel(const uint16_t
   __shared__ float s_amax[COLS];
   __shared__ __attribute__((aligned(16))) uint32_t s_tile[kTRows * (COLS / 2)];
   __shared__ int s_tmp[8];
-  __shared__ int s_seg[2];
   __shared__ GroupChunk s_gc;
   // slab-major: the blocks running together share column slabs (1-4 % faster
   // than expert-major at the Kimi shapes)

@@ -12,8 +12,8 @@
 //   bwd_dx   dx = dg w1 + du w3
 //   bwd_dw   out[e] = a_e^T b_e over expert e's rows (dw1, dw3, dw2)
 //
-// Tiles: 64 x 64 outputs, 32 of k per LDS stage, two stages; eight waves per workgroup in
-// the row modes, four in dW. What bounds fp32 is the matrix cores (a 16 x 16 x 4 MFMA
+// Tiles: 64 x 64 outputs, 32 of k per LDS stage, two stages (one in dW of few rows); eight
+// waves per workgroup in the row modes, four in dW. What bounds fp32 is the matrix cores (a 16 x 16 x 4 MFMA
 // takes 32 clocks; 154 TFLOP/s measured over a large product) and, at few tiles, how
 // evenly 64 x 64 tiles fall on the CUs, so the rest has to stay out of their way:
 // operands go to LDS by direct-to-LDS copies (16 bytes a lane, no staging registers or
@@ -161,7 +161,8 @@ __device__ __forceinline__ Seg find_segment(const int64_t* counts, int64_t R, in
   return Seg{(int)start, (int)min(cut(counts[e]), most - start)};
 }
 
-// A wave copies two of an operand's eight 1 KB pieces (8 rows, or 4 k-rows) of a stage.
+// A stage of an operand is eight 1 KB pieces (8 rows, or 4 k-rows): in the row modes a wave
+// copies one, in dW two.
 // k-contiguous: lane -> row 8 c + lane / 8, 16-byte chunk (lane & 7) ^ (row & 7)
 __device__ __forceinline__ int row_of(int c, int lane) { return 8 * c + (lane >> 3); }
 __device__ __forceinline__ int row_chunk(int lane) { return (lane & 7) ^ ((lane >> 3) & 7); }
@@ -180,8 +181,8 @@ __device__ __forceinline__ f32x2_t read_col2(const float* tile, int lane, int w,
   return *(const f32x2_t*)(tile + k * 64 + ((c ^ ((g & 1) << 3)) << 2) + 2 * (lane & 1));
 }
 
-// Row-grouped modes: 64 rows of one expert x 64 output columns. Waves: 32 x 32 each where
-// the weights are k-contiguous (gate_up, down), 16 x 64 where they are k-major (dgu, dx).
+// Row-grouped modes: 64 rows of one expert x 64 output columns, eight waves of 16 x 32. The
+// weights are k-contiguous in gate_up and down, k-major in dgu and dx.
 template <int MODE, bool ALIGNED>
 __global__ __launch_bounds__(512, MODE == kGateUp ? 6 : 8) void rows_kernel(Params p) {
   constexpr bool kTwoB = MODE == kGateUp;                 // two weights into two accumulator sets

@@ -649,11 +649,13 @@ static void launch_permute_bwd(const void* grad_routed, const void* x, const int
                                const float* scores, int64_t n_tokens, int dim, int top_k, int round_each,
                                void* grad_x, float* grad_scores, hipStream_t stream) {
   constexpr bool kRounds = sizeof(T) == 2;  // fp32 rows have no rounding between the adds
+  // (unscored fp32 rows are read as fast either way: 130 / 132 us for 537 MB)
+  constexpr bool kUnscoredStream = STREAM && sizeof(T) == 2;
   const bool round = kRounds && round_each;
   auto* kernel = scores ? (round ? permute_bwd_kernel<T, MAXK, true, kRounds, STREAM>
                                  : permute_bwd_kernel<T, MAXK, true, false, STREAM>)
-                        : (round ? permute_bwd_kernel<T, MAXK, false, kRounds, STREAM>
-                                 : permute_bwd_kernel<T, MAXK, false, false, STREAM>);
+                        : (round ? permute_bwd_kernel<T, MAXK, false, kRounds, kUnscoredStream>
+                                 : permute_bwd_kernel<T, MAXK, false, false, kUnscoredStream>);
   hipLaunchKernelGGL(kernel, dim3(stream_grid(n_tokens, 4, 16384)), dim3(256), 0, stream, (const T*)grad_routed,
                      (const T*)x, tok_pos, scores, n_tokens, dim, top_k, (T*)grad_x, grad_scores);
 }
@@ -662,8 +664,7 @@ template <typename T>
 static void launch_permute_bwd(const void* grad_routed, const void* x, const int32_t* tok_pos,
                                const float* scores, int64_t n_tokens, int dim, int top_k, int round_each,
                                void* grad_x, float* grad_scores, hipStream_t stream) {
-  // (unscored fp32 rows are read as fast either way: 130 / 132 us for 537 MB)
-  const bool nt = (scores || sizeof(T) == 2) && streamed<T>(n_tokens, dim, top_k);
+  const bool nt = streamed<T>(n_tokens, dim, top_k);
   auto* launch = top_k <= 8    ? (nt ? launch_permute_bwd<T, 8, true> : launch_permute_bwd<T, 8, false>)
                  : top_k <= 16 ? (nt ? launch_permute_bwd<T, 16, true> : launch_permute_bwd<T, 16, false>)
                                : (nt ? launch_permute_bwd<T, kMaxTopK, true> : launch_permute_bwd<T, kMaxTopK, false>);
