@@ -622,9 +622,9 @@ static int check_row_args(int64_t n_tokens, int32_t dim, int32_t top_k, int32_t 
 
 template <typename T>
 static void launch_expand(const void* src, int64_t n_tokens, int dim, int top_k, const int32_t* slot_pos,
-                          const float* scores, void* out, bool stream_stores, hipStream_t stream) {
+                          const float* scores, void* out, hipStream_t stream) {
   const dim3 grid(stream_grid(n_tokens * (dim / Chunk<T>::kN)));
-  if (stream_stores)
+  if (streamed<T>(n_tokens, dim, top_k))
     hipLaunchKernelGGL((expand_rows_kernel<T, true>), grid, dim3(256), 0, stream, (const T*)src, n_tokens, dim,
                        top_k, slot_pos, scores, (T*)out);
   else
@@ -698,11 +698,9 @@ MOE_API int moe_permute(const void* x, const int32_t* slot_pos, const float* sco
   if (n_tokens == 0) return kOk;
   if (!x || !slot_pos || !routed_input) return kErrInvalidArgument;
   if (dtype == MOE_DTYPE_BF16)
-    launch_expand<uint16_t>(x, n_tokens, dim, top_k, slot_pos, scores_sorted, routed_input,
-                            streamed<uint16_t>(n_tokens, dim, top_k), stream);
+    launch_expand<uint16_t>(x, n_tokens, dim, top_k, slot_pos, scores_sorted, routed_input, stream);
   else
-    launch_expand<float>(x, n_tokens, dim, top_k, slot_pos, scores_sorted, routed_input,
-                         streamed<float>(n_tokens, dim, top_k), stream);
+    launch_expand<float>(x, n_tokens, dim, top_k, slot_pos, scores_sorted, routed_input, stream);
   return launch_status();
 }
 
@@ -756,14 +754,11 @@ MOE_API int moe_combine_bwd(const void* grad_out, const void* routed_output, con
                                        grad_routed, grad_scores_sorted, stream);
   } else {
     if (!slot_pos) return kErrInvalidArgument;
-    // plain stores: streaming ones measure 13 % faster alone but 8 to 12 % slower in the layer step,
-    // also past kStreamBytes (us, plain | streamed: 16384 tokens of 2304, K = 8 123 | 133, of 1024
-    // 55 | 61, 8192 of 4096, K = 6 83 | 93), whose next kernel gains nothing back; 4 to 30 % slower
-    // before the permute backward, which gains about as much
+    // plain stores: streaming ones measure 13 % faster alone but 9 % slower in the layer step
     if (dtype == MOE_DTYPE_BF16)
-      launch_expand<uint16_t>(grad_out, n_tokens, dim, top_k, slot_pos, nullptr, grad_routed, false, stream);
+      launch_expand<uint16_t>(grad_out, n_tokens, dim, top_k, slot_pos, nullptr, grad_routed, stream);
     else
-      launch_expand<float>(grad_out, n_tokens, dim, top_k, slot_pos, nullptr, grad_routed, false, stream);
+      launch_expand<float>(grad_out, n_tokens, dim, top_k, slot_pos, nullptr, grad_routed, stream);
   }
   return launch_status();
 }
