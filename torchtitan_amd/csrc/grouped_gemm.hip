@@ -16,11 +16,14 @@
 //   bwd_dw2     dw2 D x H            dy^T             h^T                   tokens
 //
 // Design (gfx950, 64-wide waves):
-//  * Wave tiles of 64 x 128 (or 64 x 96) of v_mfma_f32_16x16x32_bf16 (fp32
-//    accumulate), two waves per SIMD so each hides the other's LDS latency:
-//    forward modes and dgu 4 waves / 128 x 256 block / two workgroups per CU,
-//    dx and dW 8 waves / 128 x 512, 128 x 384 or 256 x 256 block / one
-//    workgroup per CU (wider blocks copy fewer bytes per flop). k-step 32.
+//  * Tiles of v_mfma_f32_16x16x32_bf16 (fp32 accumulate), two waves per SIMD so each hides
+//    the other's LDS latency: eight waves and one workgroup per CU, or four and two. Which
+//    tile a launch takes follows from its rounds over the chip (pick_tile):
+//      gate_up, down  128 x 256 (64 x 64 waves) or 256 x 256 (64 x 128 waves), k-step 64
+//      dgu            128 x 256 of eight or of four waves, 64 x 256 of four; k-step 32
+//      dx             128 x 256 of eight or of four waves, 128 x 384, 128 x 512, gpt-oss also
+//                     256 x 256; k-step 32 (wider blocks copy fewer bytes per flop)
+//      dW             256 x 256, or 128 x 128 of four waves; k-step 32
 //  * Operands go HBM/L2 -> LDS with direct-to-LDS copies
 //    (global_load_lds_dwordx4: each wave instruction fills 1 KB of LDS), so no
 //    VGPRs stage the tiles and no ds_write is issued. Two or three LDS stages:
@@ -585,8 +588,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void grouped_gemm_kernel(GemmParams p
           __builtin_amdgcn_sched_barrier(0);
         }
       };
-      // Pipelined: the tiles with 64-wide k-steps (forward modes only). With 32-wide
-      // k-steps (the 128 x 256 forward tile, dgu, dx, dW) the plain schedule measured
+      // Pipelined: the tiles with 64-wide k-steps (the forward modes). With 32-wide
+      // k-steps (dgu, dx, dW) the plain schedule measured
       // faster. Waves with a partial row block keep the plain schedule too (their
       // conditional MFMAs with the pipeline's registers spill).
       constexpr bool kIlv = BK == 64 && decltype(full)::value;
@@ -974,15 +977,22 @@ static void launch_cfg(const GemmParams& p, int64_t R, hipStream_t stream) {
 //                  only where the wide tiles leave half the chip idle (the smaller tile
 //                  copies twice the bytes per flop: 382 -> 421 us at 1600 / 832 / 48 / 49152)
 //
-// Measured (us; D / H / experts / rows), against one fixed tile per mode with a bound on
-// the rows per expert: gate_up 2304 / 1024 / 256 / 512 399 -> 343, 16384 rows 580 -> 500,
-// 65536 950 -> 902; 7168 / 2048 / 32 / 16384 1043 -> 995; down 2048 / 1408 / 64 / 16384
-// 165 -> 128; dgu 2304 / 1024 / 256 / 16384 331 -> 289, 7168 / 2048 / 32 / 8199 458 ->
-// 400; dx 1024 / 704 / 64 / 16384 110 -> 90, 4096 / 1536 / 32 / 4096 233 -> 195; gpt-oss
-// 2880 / 2880 / 32 / 4096 gate_up 370 -> 284, down 230 -> 149, dgu 298 -> 206, dx 405 ->
-// 309; dW 256 / 512 / 8 / 8192 42 -> 24. The weights are read once whatever the tile: with
-// few rows per expert the eight-wave forward tile's three stages of whole 128-byte rows
-// keep more bytes in flight (5.2 -> 6.1 TB/s of weights at two rows per expert).
+// Measured inside forward and backward (us; D / H / experts / rows, moderately skewed), against
+// one fixed tile per mode with a bound on the rows per expert: gate_up 2304 / 1024 / 256 / 512
+// 460 -> 402, 16384 rows 573 -> 542, 65536 987 -> 886; 7168 / 2048 / 32 / 16384 1025 -> 1011;
+// down 2048 / 1408 / 64 / 16384 180 -> 135; dgu 2304 / 1024 / 256 / 16384 284 -> 278, 7168 / 2048
+// / 32 / 8199 521 -> 457, 1600 / 832 / 48 / 4096 83 -> 52; dx 1024 / 704 / 64 / 16384 128 -> 96,
+// 4096 / 1536 / 32 / 4096 238 -> 199; gpt-oss 2880 / 2880 / 32 / 4096 gate_up 394 -> 328, down
+// 222 -> 163, dgu 275 -> 203, dx 410 -> 348; dW 256 / 512 / 8 / 8192 55 -> 32 each. The weights
+// are read once whatever the tile: with few rows per expert the eight-wave forward tile's three
+// stages of whole 128-byte rows keep more bytes in flight (5.2 -> 6.1 TB/s of weights at two rows
+// per expert).
+// How far the rule is right: over 1420 shapes (2 to 65536 rows, any skew) a launch takes 0.3 to
+// 0.6 % longer than its fastest candidate in the forward modes, 4 to 6 % in dgu, 2 to 3 % in dx,
+// where the fixed tiles took 18 to 33 % longer. 2 % of the launches are over 3 % slower than on
+// the fixed tile, the worst by 43 %: the counts are not known here, and a few tiles more or less
+// than expected next to a whole number of rounds turn the choice (24 experts, 2910 rows, skewed:
+// 256 tiles of 128 rows, one round, where 313 were expected).
 enum GemmTile : int {  // rows x columns, workgroups per CU: 10000 rows + 10 columns + workgroups
   k128x256 = 1282561, k256x256 = 2562561, k128x384 = 1283841, k128x512 = 1285121,
   k64x256Two = 642562, k128x256Two = 1282562, k128x128Two = 1281282

@@ -28,9 +28,9 @@
 //    contiguous in the output row.
 // All of these reads are free of bank conflicts.
 // Measured (us, against scalar LDS reads of register-staged 16-deep tiles, four waves) at
-// 8192 rows of 8 experts, dim 256, hidden 512 | 16384 rows, 512, 1024: gate_up 59 -> 57 |
-// 330 -> 313, down 36 -> 32 | 186 -> 164, dgu 39 -> 34 | 224 -> 184, dx 64 -> 62 | 350 ->
-// 343, the three dW (one launch, before three) 123 -> 72 | 592 -> 498. Without copies and
+// 8192 rows of 8 experts, dim 256, hidden 512 | 16384 rows, 512, 1024: gate_up 59 -> 56 |
+// 329 -> 319, down 37 -> 33 | 187 -> 166, dgu 40 -> 37 | 222 -> 184, dx 67 -> 64 | 354 ->
+// 344, the three dW (one launch, before three) 157 -> 82 | 765 -> 542. Without copies and
 // stores gate_up still takes 43 | 264 us: the MFMAs at the clock they leave. Three stages
 // measured the same as two.
 // Row-grouped modes map workgroups to (expert, 64-row tile) from a scan of the counts,
